@@ -31,6 +31,7 @@ struct CarpWork {
   int64_t n = 0;
   int nshifts = 0;
   int ncolors = 0;
+  int32_t max_len = 0;               // entries of the longest row
   std::vector<int64_t> color_ptr;    // rows of colour c: rows[color_ptr[c] .. color_ptr[c+1])
   std::vector<int64_t> color_chunk;  // first chunk of colour c
   std::vector<int32_t> h_rows;
@@ -48,58 +49,125 @@ struct CarpCoef {
   T sr[kCarpCols], si[kCarpCols], w[kCarpCols];
 };
 
-template <typename T, bool RC>
+// One colour.  A lane owns VPL consecutive columns of X (a 16-byte vector
+// where the layout allows) in one row, nvec / VPL lanes per row.  A row's
+// entries are taken in batches of LB: all of a batch's indices and values go
+// out together, then all its x rows, so a row of up to LB entries (ONE: every
+// row of the matrix) costs three dependent round trips - row data, entries, x
+// - whatever its length, and its entries and x rows stay in registers for the
+// projection.  Rows of one colour have no x entry in common, so a launch
+// reuses nothing but the other half of a cache line; each XCD takes a
+// contiguous range of the colour's rows to keep that half in its L2.
+// What bounds it: the round trips of a launch (a colour of 55k rows is one
+// wave of workgroups) and the x lines read and written once per colour.
+// 1024 x 1024 graphene sheet with 13 entries per row, 8 columns, FP64, 19
+// colours: 41 -> 25 us a launch, 1571 -> 963 us a sweep against one lane per
+// (row, column) that read entry after entry and read all of them twice.
+// A column that a row stores more than once (the entries are sorted, so the
+// repeats are neighbours) continues from the value the entry before it wrote,
+// and the diagonal entry from the x_i that the shift term has updated.
+template <typename T, bool RC, int VPL, int LB, bool ONE>
 __global__ void __launch_bounds__(kBlock)
     k_kacz(const int32_t* __restrict__ rows, const int32_t* __restrict__ rlen, const int64_t* __restrict__ cptr,
-           int64_t nr, const int32_t* __restrict__ ci, const T* __restrict__ va, int nvec, const CarpCoef<T> coef,
-           const T* __restrict__ b, int64_t ldb, T* xr, T* xi, int64_t ldx) {
-  const int64_t total = nr * nvec;
-  for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < total; e += (int64_t)gridDim.x * kBlock) {
-    const int64_t r = e / nvec;
-    const int c = (int)(e - r * nvec);
+           int64_t nr, int64_t ntiles, const int32_t* __restrict__ ci, const T* __restrict__ va, int lpr,
+           const CarpCoef<T> coef, const T* __restrict__ b, int64_t ldb, T* xr, T* xi, int64_t ldx) {
+  const uint32_t rpt = kBlock / (uint32_t)lpr;  // rows per tile (lanes beyond rpt * lpr stay idle)
+  const uint32_t rl = threadIdx.x / (uint32_t)lpr;
+  if (rl >= rpt) return;
+  const int c0 = (int)(threadIdx.x - rl * (uint32_t)lpr) * VPL;
+  T s_r[VPL], s_i[VPL], w[VPL];
+#pragma unroll
+  for (int e = 0; e < VPL; e++) {
+    s_r[e] = coef.sr[c0 + e];
+    s_i[e] = RC ? coef.si[c0 + e] : T(0);
+    w[e] = coef.w[c0 + e];
+  }
+  const TileWalk tw = xcd_tiles(ntiles);
+  for (int64_t t = tw.t; t < tw.end; t += tw.stride) {
+    const int64_t r = t * rpt + rl;
+    if (r >= nr) continue;
     const int64_t i = rows[r];
     const int len = rlen[r];
     const int64_t k0 = cptr[r / kCarpChunk] + (r % kCarpChunk);
-    const T s_r = coef.sr[c], s_i = RC ? coef.si[c] : T(0), w = coef.w[c];
-    const T xri = xr[i * ldx + c];
-    T tr, ti = T(0);
-    if (RC) {
-      const T xii = xi[i * ldx + c];
-      tr = fma(s_i, xii, -s_r * xri);
-      ti = fma(-s_i, xri, -s_r * xii);
-    } else {
-      tr = -s_r * xri;
+    T xri[VPL], xii[VPL], bv[VPL], tr[VPL], ti[VPL];
+    vload<T, VPL>(xr + i * ldx + c0, xri);
+    if (RC) vload<T, VPL>(xi + i * ldx + c0, xii);
+    if (b) vload<T, VPL>(b + i * ldb + c0, bv);
+    int32_t cj[LB];
+    T a[LB], xg[LB][VPL], yg[RC ? LB : 1][VPL];
+    auto load = [&](int q0) {
+#pragma unroll
+      for (int q = 0; q < LB; q++)
+        if (q0 + q < len) {
+          cj[q] = ci[k0 + (int64_t)(q0 + q) * kCarpChunk];
+          a[q] = va[k0 + (int64_t)(q0 + q) * kCarpChunk];
+        }
+#pragma unroll
+      for (int q = 0; q < LB; q++)
+        if (q0 + q < len) {
+          vload<T, VPL>(xr + (int64_t)cj[q] * ldx + c0, xg[q]);
+          if constexpr (RC) vload<T, VPL>(xi + (int64_t)cj[q] * ldx + c0, yg[q]);
+        }
+    };
+#pragma unroll
+    for (int e = 0; e < VPL; e++) {
+      if (RC) {
+        tr[e] = fma(s_i[e], xii[e], -s_r[e] * xri[e]);
+        ti[e] = fma(-s_i[e], xri[e], -s_r[e] * xii[e]);
+      } else {
+        tr[e] = -s_r[e] * xri[e];
+      }
     }
-    T d = T(0), nrm = T(0);
-    for (int q = 0; q < len; q++) {
-      const int64_t k = k0 + (int64_t)q * kCarpChunk;
-      const int64_t j = ci[k];
-      const T a = va[k];
-      tr = fma(a, xr[j * ldx + c], tr);
-      if (RC) ti = fma(a, xi[j * ldx + c], ti);
-      nrm = fma(a, a, nrm);
-      if (j == i) d = a;
+    T d = T(0), nrm0 = T(0);
+    for (int q0 = 0; q0 < (ONE ? 1 : len); q0 += LB) {
+      load(q0);
+#pragma unroll
+      for (int q = 0; q < LB; q++)
+        if (q0 + q < len) {
+#pragma unroll
+          for (int e = 0; e < VPL; e++) {
+            tr[e] = fma(a[q], xg[q][e], tr[e]);
+            if constexpr (RC) ti[e] = fma(a[q], yg[q][e], ti[e]);
+          }
+          nrm0 = fma(a[q], a[q], nrm0);
+          if (cj[q] == i) d = a[q];
+        }
     }
-    if (b) tr = tr - b[i * ldb + c];
-    nrm = fma(s_r, s_r, fma(T(-2) * d, s_r, nrm));
-    if (RC) nrm = fma(s_i, s_i, nrm);
-    if (nrm == T(0)) nrm = T(1);
-    tr = (tr * w) / nrm;
-    if (RC) ti = (ti * w) / nrm;
-    // projection: the shift term of x_i first, then every column of the row
-    if (RC) {
-      const T xii = xi[i * ldx + c];
-      xr[i * ldx + c] = xri + fma(ti, s_i, tr * s_r);
-      xi[i * ldx + c] = xii + fma(-tr, s_i, ti * s_r);
-    } else {
-      xr[i * ldx + c] = fma(tr, s_r, xri);
+#pragma unroll
+    for (int e = 0; e < VPL; e++) {
+      if (b) tr[e] = tr[e] - bv[e];
+      T nrm = fma(s_r[e], s_r[e], fma(T(-2) * d, s_r[e], nrm0));
+      if (RC) nrm = fma(s_i[e], s_i[e], nrm);
+      if (nrm == T(0)) nrm = T(1);
+      tr[e] = (tr[e] * w[e]) / nrm;
+      if (RC) ti[e] = (ti[e] * w[e]) / nrm;
+      // projection: the shift term of x_i first, then every column of the row
+      if (RC) {
+        xri[e] = xri[e] + fma(ti[e], s_i[e], tr[e] * s_r[e]);
+        xii[e] = xii[e] + fma(-tr[e], s_i[e], ti[e] * s_r[e]);
+      } else {
+        xri[e] = fma(tr[e], s_r[e], xri[e]);
+      }
     }
-    for (int q = 0; q < len; q++) {
-      const int64_t k = k0 + (int64_t)q * kCarpChunk;
-      const int64_t j = ci[k];
-      const T a = va[k];
-      xr[j * ldx + c] = fma(-tr, a, xr[j * ldx + c]);
-      if (RC) xi[j * ldx + c] = fma(-ti, a, xi[j * ldx + c]);
+    vstore<T, VPL>(xr + i * ldx + c0, xri);
+    if (RC) vstore<T, VPL>(xi + i * ldx + c0, xii);
+    int32_t jp = -1;
+    T px[VPL], py[VPL];  // what the entry before wrote, to column jp
+    for (int q0 = 0; q0 < (ONE ? 1 : len); q0 += LB) {
+      if (!ONE) load(q0);
+#pragma unroll
+      for (int q = 0; q < LB; q++)
+        if (q0 + q < len) {
+          const bool again = cj[q] == jp, own = cj[q] == i;
+#pragma unroll
+          for (int e = 0; e < VPL; e++) {
+            px[e] = fma(-tr[e], a[q], again ? px[e] : (own ? xri[e] : xg[q][e]));
+            if constexpr (RC) py[e] = fma(-ti[e], a[q], again ? py[e] : (own ? xii[e] : yg[q][e]));
+          }
+          jp = cj[q];
+          vstore<T, VPL>(xr + (int64_t)cj[q] * ldx + c0, px);
+          if constexpr (RC) vstore<T, VPL>(xi + (int64_t)cj[q] * ldx + c0, py);
+        }
     }
   }
 }
@@ -176,6 +244,7 @@ void* carp_setup(const SparseMat<T>* A, int nshifts) {
         rlen[r] = (int32_t)(A->crs_ptr[i + 1] - A->crs_ptr[i]);
         wmax = std::max(wmax, rlen[r]);
       }
+      W->max_len = std::max(W->max_len, wmax);
       cptr.push_back(slots);
       slots += (int64_t)wmax * kCarpChunk;
     }
@@ -224,6 +293,39 @@ void carp_destroy(void* work) {
   delete W;
 }
 
+template <typename T, bool RC, int VPL, int LB, bool ONE, typename... Args>
+void kacz_go(const int32_t* rows, const int32_t* rlen, const int64_t* cptr, int64_t nr, const int32_t* ci, const T* va,
+             int lpr, Args... args) {
+  const int64_t rpt = kBlock / lpr, ntiles = (nr + rpt - 1) / rpt;
+  const int grid = persistent_blocks(k_kacz<T, RC, VPL, LB, ONE>, 0, ntiles);
+  hipLaunchKernelGGL((k_kacz<T, RC, VPL, LB, ONE>), dim3(grid), dim3(kBlock), 0, rt().stream, rows, rlen, cptr, nr,
+                     ntiles, ci, va, lpr, args...);
+  PHX_HIP(hipGetLastError());
+}
+
+// one colour on nc columns: vector lanes where every block's rows are whole
+// 16-byte vectors (real shifts; the complex update holds twice the values),
+// and the batch that takes the longest row at once, up to 16 entries
+template <typename T>
+void kacz_launch(const int32_t* rows, const int32_t* rlen, const int64_t* cptr, int64_t nr, int32_t max_len,
+                 const int32_t* ci, const T* va, int nc, const CarpCoef<T>& coef, const T* b, int64_t ldb, T* xr,
+                 T* xi, int64_t ldx) {
+  constexpr int V = 16 / sizeof(T);
+  auto al = [](const T* p, int64_t ld) { return ((uintptr_t)p & 15) == 0 && ld % V == 0; };
+  const bool vec = !xi && nc % V == 0 && al(xr, ldx) && (!b || al(b, ldb));
+#define PHX_KACZ(RC, VPL)                                                                                            \
+  (max_len <= 8    ? kacz_go<T, RC, VPL, 8, true>(rows, rlen, cptr, nr, ci, va, nc / VPL, coef, b, ldb, xr, xi, ldx)  \
+   : max_len <= 16 ? kacz_go<T, RC, VPL, 16, true>(rows, rlen, cptr, nr, ci, va, nc / VPL, coef, b, ldb, xr, xi, ldx) \
+                   : kacz_go<T, RC, VPL, 8, false>(rows, rlen, cptr, nr, ci, va, nc / VPL, coef, b, ldb, xr, xi, ldx))
+  if (xi)
+    PHX_KACZ(true, 1);
+  else if (vec)
+    PHX_KACZ(false, V);
+  else
+    PHX_KACZ(false, 1);
+#undef PHX_KACZ
+}
+
 // forward then backward sweep over the colours; B may be null (b = 0),
 // si and Xi null for real shifts
 template <typename T>
@@ -238,7 +340,6 @@ void carp_sweep(const SparseMat<T>* A, void* work, const T* sr, const T* si, con
               "vector shapes do not match the matrix");
   PHX_REQUIRE(!Xi || (Xi->nrows == W->n && Xi->nvec == nvec && Xi->lda == Xr->lda), PHIST_INVALID_INPUT,
               "X_i must match X_r");
-  hipStream_t st = rt().stream;
   ktimer_begin();  // whole sweep (all colour launches) when the kernel timer is on
   // columns are independent: blocks of up to kCarpCols columns sweep one after another
   for (int c0 = 0; c0 < nvec; c0 += kCarpCols) {
@@ -256,16 +357,8 @@ void carp_sweep(const SparseMat<T>* A, void* work, const T* sr, const T* si, con
     auto run = [&](int c) {
       const int64_t r0 = W->color_ptr[c], nr = W->color_ptr[c + 1] - r0;
       if (nr == 0) return;
-      const int64_t total = nr * nc;
-      const int grid = (int)std::min<int64_t>((total + kBlock - 1) / kBlock, (int64_t)rt().num_cu * 8);
-      const int64_t* cp = W->chunk_ptr + W->color_chunk[c];
-      if (xi)
-        hipLaunchKernelGGL((k_kacz<T, true>), dim3(grid), dim3(kBlock), 0, st, W->rows + r0, W->rlen + r0, cp, nr,
-                           W->col, W->val, nc, coef, bp, ldb, xr, xi, Xr->lda);
-      else
-        hipLaunchKernelGGL((k_kacz<T, false>), dim3(grid), dim3(kBlock), 0, st, W->rows + r0, W->rlen + r0, cp, nr,
-                           W->col, W->val, nc, coef, bp, ldb, xr, (T*)nullptr, Xr->lda);
-      PHX_HIP(hipGetLastError());
+      kacz_launch<T>(W->rows + r0, W->rlen + r0, W->chunk_ptr + W->color_chunk[c], nr, W->max_len, W->col, W->val, nc,
+                     coef, bp, ldb, xr, xi, Xr->lda);
     };
     for (int c = 0; c < W->ncolors; c++) run(c);
     for (int c = W->ncolors - 1; c >= 0; c--) run(c);

@@ -241,6 +241,39 @@ def test_sweep_empty_rows(be64):
     A.delete()
 
 
+@pytest.mark.parametrize("nvec,rc", [(1, False), (3, False), (8, False), (66, False), (2, True)])
+@pytest.mark.parametrize("longest", [1, 8, 9, 16, 17, 40])
+def test_sweep_row_lengths(be64, be32, longest, nvec, rc):
+    """rows of 0 .. longest entries around the sizes of the batches a row is
+    taken in, with and without a diagonal entry, some columns stored two or
+    three times"""
+    rng = np.random.default_rng(100 * longest + nvec)
+    n = 120
+    made = []
+    for i in range(n):
+        k = longest if i % 7 == 0 else int(rng.integers(0, longest + 1))
+        cols = rng.integers(0, n, k)
+        if k >= 4 and i % 3 == 0:
+            cols[1] = cols[2] = cols[0]  # a repeated column
+        if k >= 2 and i % 2 == 0:
+            cols[-1] = i
+        if k >= 6 and i % 4 == 0:
+            cols[-2] = i  # the diagonal twice
+        made.append((cols.tolist(), rng.uniform(-1, 1, k).tolist()))
+    rf = rowfunc_of(ol.crs_from_rows(n, n, made))
+    sr, om = rng.uniform(-1, 1, nvec), rng.uniform(0.5, 1.9, nvec)
+    si = rng.uniform(0.1, 1, nvec) if rc else None
+    A = be64.from_rowfunc(n, longest, rf, None)
+    got, goti, want, wanti, _ = run_pair(be64, A, nvec, sr, om, si=si, seed=longest)
+    assert np.array_equal(got, want) and (not rc or np.array_equal(goti, wanti))
+    A.delete()
+    if not rc:
+        A = be32.laplace3d(9, 8, 7) if longest == 8 else be32.banded_random(300, min(longest, 30), 40, 40.0, 3)
+        got, _, want, _, _ = run_pair(be32, A, nvec, sr, om, seed=longest)
+        assert np.array_equal(got, want)
+        A.delete()
+
+
 def test_setup_rejects_rectangular(be64):
     import phist_amd
     rows = ol.crs_from_rows(5, 8, [([0], [1.0]), ([1, 7], [1.0, 2.0]), ([2], [1.0]), ([3], [1.0]), ([4], [1.0])])
