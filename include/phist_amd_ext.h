@@ -24,28 +24,29 @@ void phist_amd_sparseMat_set_format(int C, int sigma, int* iflag);
  * resident wave of workgroups on every CU) */
 void phist_amd_set_grid_blocks(int nblocks, int* iflag);
 /* workgroups per CU of the SpMV's persistent grid (0 = as many as fit;
- * n < 0 = the built-in table, the default: 2 for rows of >= 24 nonzeros and
- * blocks of >= 4 columns, whose gathers then keep a wide band's x rows
- * L2-resident, 3 for such rows and narrower blocks, 6 for shorter rows) */
+ * n < 0 = the default: the matrix's tuned value, else a rule by the rows'
+ * length, the block width and the distance of the entries from the diagonal) */
 void phist_amd_set_spmv_blocks_per_cu(int n, int* iflag);
 /* bytes of a block row each lane of the SpMV gathers per nonzero (0 = the
- * default, one 16-byte vector; sizeof(scalar) = one scalar per lane; 32 or 64
- * = two or four 16-byte vectors per lane, taken when the block width and
- * leading dimension are multiples of that many scalars).  Every choice gives
+ * default: the matrix's tuned value, else one or two 16-byte vectors by a
+ * rule as for the workgroups; sizeof(scalar) = one scalar per lane; 32 or 64
+ * = two or four 16-byte vectors per lane, taken when the block width is a
+ * multiple of that many scalars and the block smaller than 4 GiB).  Every choice gives
  * the same result bit for bit: a row's sum is always formed by the lane that
  * owns its columns, in the row's entry order. */
 void phist_amd_set_spmv_lane_bytes(int bytes, int* iflag);
 /* entries of a row whose val/col loads and x gathers the SpMV issues
  * together before their multiply-adds (0 = the default: the matrix's tuned
- * value, else 8; 8, 16 or 32).  16 and 32 also request the next batch's
- * val/col before the current batch's gathers; they apply to row groups of at
- * most 8 lanes gathering at most 32 bytes each, without per-column x
- * factors, and fall back to 8 otherwise.  Every choice
- * gives the same result bit for bit. */
+ * value, else 8 or 16 by a rule; 8, 16 or 32).  16 (and 32, the same) applies
+ * to plain products of rows shorter than 24 entries, in row groups of at most
+ * 8 lanes gathering at most 32 bytes each; elsewhere 8, and 4 for matrices
+ * whose longest row has at most 4 entries.  Every choice gives the same
+ * result bit for bit. */
 void phist_amd_set_spmv_depth(int slots, int* iflag);
 /* block columns per SpMV launch: ncols > 0 = at most that many (a multiple of
  * the scalars each lane holds, else ignored), 0 = as many as 64 lane groups
- * hold, -1 = the default: the matrix's tuned value, else 0.  Each further
+ * hold, -1 = the default: the matrix's tuned value, else 128 bytes of columns
+ * for rows of at least 24 entries and 0 for shorter ones.  Each further
  * launch reads the matrix again; wide rows of x (256-byte rows at 32 FP64
  * columns) gather half as many bytes per launch in two blocks of 16.  Every
  * choice gives the same result bit for bit (column dots to rounding). */
@@ -77,8 +78,8 @@ void phist_amd_spmv_staged_launches(int64_t* count, int* iflag);
 /* SpMV autotuner.  For each block width nvecs[0..n_nvec) (1..256, at most 16
  * widths) it times the product y = A*x on the device over the gather width
  * per lane (one scalar, or one, two or four 16-byte vectors: how many lanes
- * share a row), the workgroups per CU (1, 2, 3, 4, 6, 8), for rows of at
- * least 16 entries the depth (8, 16 or 32, phist_amd_set_spmv_depth), for more
+ * share a row), the workgroups per CU (1, 2, 3, 4, 6, 8), for rows of 9 to
+ * 23 entries the depth (8 or 16, phist_amd_set_spmv_depth), for more
  * than 16 columns launches of 16 (and of 32 above 32) columns
  * (phist_amd_set_spmv_col_block), where the matrix allows it x staged in LDS
  * per workgroup tile (phist_amd_set_spmv_stage), and with

@@ -314,20 +314,33 @@ template <typename T> void sd_from_device_async(const SdMat<T>* M);
 // launch settings of the SpMV for one matrix and block width: bytes each
 // lane gathers per nonzero (0 = one 16-byte vector) and workgroups per CU
 // (0 = as many as fit)
-// the depth the SpMV runs for a requested depth (8, 16 or 32), the scalars
-// per lane vpl, the scalar size and the block width: 16 and 32 need at most
-// 32 gathered bytes per lane and at most 8 lanes per row; otherwise 8
+// the block columns a lane of the SpMV holds for a block of nvec columns and
+// lane bytes lb (a setting; 0: the default): one column for lb up to one
+// scalar, two or four 16-byte vectors for 32 and 64 where they divide the
+// block, else one vector (two columns or one of narrower blocks)
+template <typename T>
+inline int spmv_lane_columns(int nvec, int lb) {
+  constexpr int V16 = 16 / sizeof(T);
+  if (lb > 0 && lb <= (int)sizeof(T)) return 1;
+  const int w = lb / (int)sizeof(T);
+  if ((w == 2 * V16 || w == 4 * V16) && nvec % w == 0) return w;
+  return nvec >= V16 ? V16 : nvec >= 2 ? 2 : 1;
+}
+
+// the depth the SpMV runs for a requested depth, the scalars per lane vpl,
+// the scalar size and the block width: 16 needs at most 32 gathered bytes per
+// lane and at most 8 lanes per row; otherwise 8
 inline int spmv_effective_depth(int depth, int vpl, int scalar_bytes, int ncols) {
   int groups = (std::min(ncols, 64 * vpl) + vpl - 1) / vpl, lpr = 1;
   while (lpr < groups) lpr <<= 1;
   if (lpr > 8 || vpl * scalar_bytes > 32) return 8;
-  return depth >= 32 ? 32 : (depth >= 16 ? 16 : 8);
+  return depth >= 16 ? 16 : 8;
 }
 
 struct SpmvTuned {
   int lane_bytes = 0;
   int blocks_per_cu = 0;
-  int depth = 8;  // entries per row whose loads are issued together (8 or 32)
+  int depth = 8;  // entries per row whose loads are issued together
   int col_block = 0;  // block columns per launch (0: as many as 64 lane groups hold)
   int stage = 0;      // x rows of each tile staged in LDS
   double ms = 0.0;  // measured time per product when chosen
@@ -376,6 +389,7 @@ struct SparseMat {
   int32_t* d_col = nullptr;        // [nnz_padded] column of each slot
   T* d_val = nullptr;              // [nnz_padded] value of each slot
   bool perm_identity = true;
+  double gather_span = 0.0;  // mean distance of a sample of the entries from the diagonal (rows)
   // host copies of the SELL index arrays (for inspection)
   std::vector<int64_t> h_chunk_ptr;
   std::vector<int32_t> h_chunk_w;

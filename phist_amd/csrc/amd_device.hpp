@@ -60,6 +60,18 @@ __device__ inline void vstore(T* p, const T (&in)[N]) {
   }
 }
 
+// vload / vstore at any address aligned for one scalar
+template <typename T, int N>
+struct alignas(sizeof(T)) VecU {
+  T v[N];
+};
+template <typename T, int N>
+__device__ inline void uload(const T* p, T (&out)[N]) {
+  const VecU<T, N> t = *reinterpret_cast<const VecU<T, N>*>(p);
+#pragma unroll
+  for (int e = 0; e < N; e++) out[e] = t.v[e];
+}
+
 // vstore with non-temporal stores (the written lines are not kept in the
 // caches): 16-byte vectors where N scalars make whole vectors, else scalars
 template <typename T, int N>
@@ -77,6 +89,35 @@ __device__ inline void vstore_nt(T* p, const T (&in)[N]) {
   } else {
 #pragma unroll
     for (int e = 0; e < N; e++) __builtin_nontemporal_store(in[e], p + e);
+  }
+}
+
+// the elements from `own` on of in[0..N) to p (at any address aligned for one
+// scalar): the whole vector where own is 0, else one by one
+template <typename T, int N>
+__device__ inline void put_owned(T* p, const T (&in)[N], int own, bool nt) {
+  if (own == 0) {
+    if (nt) {
+      typedef T vec_t __attribute__((ext_vector_type(N == 1 ? 2 : N)));
+      typedef vec_t vecu_t __attribute__((aligned(sizeof(T))));
+      if constexpr (N == 1) {
+        __builtin_nontemporal_store(in[0], p);
+      } else {
+        vec_t v;
+#pragma unroll
+        for (int e = 0; e < N; e++) v[e] = in[e];
+        __builtin_nontemporal_store(v, reinterpret_cast<vecu_t*>(p));
+      }
+    } else {
+      VecU<T, N> t;
+#pragma unroll
+      for (int e = 0; e < N; e++) t.v[e] = in[e];
+      *reinterpret_cast<VecU<T, N>*>(p) = t;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; e++)
+      if (e >= own) p[e] = in[e];
   }
 }
 

@@ -12,8 +12,7 @@
 // new block (fused_spmv_mvTmv, :68) on the matrix cores.
 //
 // Mapping onto CDNA4: a row is owned by LPR lanes of one wave64, each lane
-// holding VPL consecutive block columns (16-byte vectors where the layout
-// allows), so a wave covers 64/LPR consecutive SELL rows and the x gather of
+// holding VPL consecutive block columns (16-byte vectors or more), so a wave covers 64/LPR consecutive SELL rows and the x gather of
 // one nonzero is one contiguous LPR*VPL*sizeof(T) segment.  val/col are read
 // coalesced from the column-major chunk layout with non-temporal loads, so
 // the L2 keeps the x rows being gathered.  The grid is persistent and
@@ -32,7 +31,7 @@ struct SpmvArgs {
   const int32_t* __restrict__ col;
   const T* __restrict__ val;
   int clog2;
-  int64_t nslots;
+  int64_t nrows, nslots;
   int64_t ntiles;
   const T* __restrict__ x;
   int64_t ldx;
@@ -41,13 +40,15 @@ struct SpmvArgs {
   T* __restrict__ u;
   int64_t ldu;
   int ncols;  // block columns handled by this launch
+  bool x64;   // host side: x offsets need 64 bits
+  bool full;  // host side: the instance with epilogues
   int nact;   // lanes of columns >= nact skip their loads and stores (same kernel, grid and sums)
   T alpha, beta, gamma, delta;
   int flags;
   int blocks_per_cu;  // host side: persistent grid size per CU (0 = as many as fit)
   T* __restrict__ partials;  // [gridDim.x][2][ncols]
   const T* __restrict__ shift_dev;  // shifts on the device (this launch's columns), else shift[]
-  const double* __restrict__ xscale;  // per-column factors of x (XSC kernels), stride xscale_stride
+  const double* __restrict__ xscale;  // per-column factors of x (may be null), stride xscale_stride
   int64_t xscale_stride;
   // staged kernels: the tile's column intervals and each slot's window row
   // (SellStage), 16-byte pieces per window row (st_ppr) and log2 of the
@@ -60,11 +61,9 @@ struct SpmvArgs {
   T shift[64 * 4];
 };
 
-// Workgroups per CU by row length and block width, from a measured sweep
-// (1..8 per CU on MI355X; FP64, nvec 1..16; banded 32-nnz rows, XXZ chain,
-// 3D Laplacian, honeycomb sheets): long rows gathered from a wide band run
-// best with few workgroups (the gathered x rows stay in L2), short rows need
-// more waves in flight to cover the gather latency.
+// Workgroups per CU of the staged and Gram kernels by row length and block
+// width, from a measured sweep (1..8 per CU on MI355X; FP64, nvec 1..16;
+// banded 32-nnz rows, XXZ chain, 3D Laplacian, honeycomb sheets).
 inline int spmv_table_blocks_per_cu(double nnz_per_row, int nvec) {
   if (nnz_per_row >= 24.0) return nvec >= 4 ? 2 : 3;
   if (nnz_per_row >= 16.0) return 4;
@@ -136,6 +135,217 @@ __device__ inline T group_bcast_t(T v, int src, int lane) {
   }
 }
 
+// The products without a Gram epilogue or staged x.  A row belongs to LPR
+// lanes that hold VPL consecutive block columns each; the last lane's window
+// moves back so that it ends with the row (any width of at least VPL columns
+// reads whole vectors, at the scalars' own alignment), and of the columns two
+// lanes then hold only the first lane stores and counts.  The lanes of a row
+// load its val/col together (lane q takes slot j = jb*LPR + q, coalesced over
+// the rows of the chunk) and share them by group broadcast.
+//
+// A batch covers SL entries of a row.  What bounds short rows is the chain of
+// dependent loads - chunk metadata, indices, x rows - with few bytes under
+// way at each link; what covers it is waves, so the kernel is built to hold
+// few registers: indices and x rows are addressed by 32-bit offsets from
+// scalar bases, a value is broadcast where it is used, the plain product
+// (FULL = false) carries no epilogue state, and a batch is no longer than the
+// matrix's rows (SL 4 for a sheet).  Inside a long row the next batch's
+// indices are requested before this batch's gathers; y (beta != 0) and x's own
+// row come with the first.  Beyond the L1 each gather moves a 128-byte
+// line from the L2, which is what bounds wide bands and chains.
+// Measured (us, the kernel before this one -> this one, default launches):
+// sheet 1499 x 1001, 5 FP64 columns 94.7 -> 45; sheet 2000 x 4000, 32 columns
+// 1968 -> 1092; 24-spin chain, 4 FP32 columns 147 -> 106, 1 FP64 column 153 ->
+// 121; 128^3 Laplacian, 1 column 51.8 -> 40.4, 16 columns 225 -> 213; 4.2 M
+// rows x 32 in a band of +-50k, 8 columns 1242 -> 1001, 32 columns 4962 ->
+// 3280 (floors by the byte model at 5.5 TB/s: 35, 815, 68, 86, 38, 129, 390
+// and 683).
+template <typename T, int VPL, int LPR, int SL, bool FULL, bool X64>
+__global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
+  constexpr int RPW = 64 / LPR;
+  constexpr int RPB = (kBlock / 64) * RPW;
+  constexpr int KB = SL > LPR ? SL / LPR : 1;  // val/col loads per lane and batch
+  constexpr int BATCH = KB * LPR;              // slots per batch and row
+  constexpr int SUBMAX = VPL * (int)sizeof(T) > 32 ? 8 : 16;
+  constexpr int SUB = BATCH < SUBMAX ? BATCH : SUBMAX;  // gathers issued before their FMAs
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane % LPR;
+  const int rw = lane / LPR;
+  const int c0 = min(q * VPL, a.ncols - VPL);
+  const int own = q * VPL - c0;  // columns of this lane's window that the lane before it holds as well
+  const bool colok = q * VPL < a.nact;
+  const int flags = FULL ? a.flags : (a.flags & F_NTY);
+
+  T sh[VPL], dww[VPL], dvw[VPL];
+#pragma unroll
+  for (int e = 0; e < VPL; e++) {
+    sh[e] = (colok && (flags & F_SHIFT)) ? (a.shift_dev ? a.shift_dev[c0 + e] : a.shift[c0 + e]) : T(0);
+    dww[e] = dvw[e] = T(0);
+  }
+  // x row of column cc: byte offsets of 32 bits from a.x unless the block is larger (X64)
+  const uint32_t xld = (uint32_t)(a.ldx * (int64_t)sizeof(T)), xc0 = (uint32_t)c0 * (uint32_t)sizeof(T);
+  auto gather = [&](int32_t cc, T (&out)[VPL]) {
+    if constexpr (X64)
+      uload<T, VPL>(a.x + (int64_t)cc * a.ldx + c0, out);
+    else
+      uload<T, VPL>(reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.x) + ((uint32_t)cc * xld + xc0)), out);
+  };
+
+  // a row's chunk width and the slot of its first entry, from the first slot
+  // of the chunk the wave's rows begin in
+  struct Tile {
+    const T* val;
+    const int32_t* col;
+    int32_t w;
+    uint32_t off;
+  };
+  const TileWalk tw = xcd_tiles(a.ntiles);
+  auto tile = [&](int64_t t) {
+    const int64_t s0 = t * RPB + wv * RPW, s = s0 + rw;
+    Tile m{nullptr, nullptr, 0, 0};
+    if (t < tw.end && s0 < a.nslots) {
+      const int64_t first = a.chunk_ptr[s0 >> a.clog2];
+      m.val = a.val + first;
+      m.col = a.col + first;
+      if (s < a.nslots) {
+        m.w = a.chunk_w[s >> a.clog2];
+        m.off = (uint32_t)(a.chunk_ptr[s >> a.clog2] - first) + (uint32_t)(s & ((1 << a.clog2) - 1));
+      }
+    }
+    return m;
+  };
+  // val/col of the batch starting at entry j0 (0 / column 0 beyond the row)
+  auto load_batch = [&](const Tile& m, int j0, T (&v)[KB], int32_t (&cj)[KB]) {
+#pragma unroll
+    for (int u = 0; u < KB; u++) {
+      const int j = j0 + u * LPR + q;
+      v[u] = T(0);
+      cj[u] = 0;
+      if (j < m.w) {
+        const uint32_t slot = m.off + ((uint32_t)j << a.clog2);
+        v[u] = __builtin_nontemporal_load(m.val + slot);
+        cj[u] = __builtin_nontemporal_load(m.col + slot);
+      }
+    }
+  };
+
+  T v[KB];
+  int32_t cj[KB];
+  for (int64_t t = tw.t; t < tw.end; t += tw.stride) {
+    // all lanes stay in the loop body (group broadcasts need every lane)
+    const Tile cur = tile(t);
+    const int64_t s = t * RPB + wv * RPW + rw;
+    int32_t row = -1;
+    if (a.perm) {
+      if (s < a.nslots) row = a.perm[s];
+    } else if (s < a.nrows) {
+      row = (int32_t)s;
+    }
+    const bool live = row >= 0 && colok;
+    T acc[VPL], xo[VPL], yo[VPL];
+#pragma unroll
+    for (int e = 0; e < VPL; e++) xo[e] = yo[e] = T(0);
+    if (FULL && live && (flags & (F_SHIFT | F_DVW))) gather(row, xo);
+    if (FULL && live && (flags & F_BETA)) uload<T, VPL>(a.y + (int64_t)row * a.ldy + c0, yo);
+#pragma unroll
+    for (int e = 0; e < VPL; e++) acc[e] = (flags & F_SHIFT) ? sh[e] * xo[e] : T(0);
+
+    load_batch(cur, 0, v, cj);
+    for (int j0 = 0; __any(j0 < cur.w);) {
+      const bool more = __any(j0 + BATCH < cur.w);  // uniform over the wave
+      T vn[KB];
+      int32_t cn[KB];
+      if (more) load_batch(cur, j0 + BATCH, vn, cn);
+      // slot j0+k of this row sits in lane k % LPR of the group, register k / LPR
+#pragma unroll
+      for (int k0 = 0; k0 < BATCH; k0 += SUB) {
+        T xg[SUB][VPL];
+#pragma unroll
+        for (int kk = 0; kk < SUB; kk++) {
+          const int k = k0 + kk;
+          const int32_t cc = group_bcast<LPR>(cj[k / LPR], k % LPR, lane);
+          if (colok && (j0 + k) < cur.w) gather(cc, xg[kk]);
+        }
+#pragma unroll
+        for (int kk = 0; kk < SUB; kk++) {
+          const int k = k0 + kk;
+          const T vk = group_bcast_t<LPR>(v[k / LPR], k % LPR, lane);
+          if (colok && (j0 + k) < cur.w) {
+#pragma unroll
+            for (int e = 0; e < VPL; e++) acc[e] = fma(vk, xg[kk][e], acc[e]);
+          }
+        }
+      }
+      if (!more) break;
+      j0 += BATCH;
+#pragma unroll
+      for (int u = 0; u < KB; u++) {
+        v[u] = vn[u];
+        cj[u] = cn[u];
+      }
+    }
+
+    if (live) {
+      T yn[VPL];
+      if (FULL && a.xscale) {  // (A + s)(x .* f) = ((A + s) x) .* f, one product per result
+#pragma unroll
+        for (int e = 0; e < VPL; e++) {
+          const T f = (T)a.xscale[(int64_t)(c0 + e) * a.xscale_stride];
+          acc[e] *= f;
+          xo[e] *= f;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < VPL; e++) yn[e] = (flags & F_BETA) ? fma(a.alpha, acc[e], a.beta * yo[e]) : a.alpha * acc[e];
+      put_owned<T, VPL>(a.y + (int64_t)row * a.ldy + c0, yn, own, flags & F_NTY);
+      if (flags & F_DWW) {
+#pragma unroll
+        for (int e = 0; e < VPL; e++) dww[e] = fma(yn[e], yn[e], dww[e]);
+      }
+      if (flags & F_DVW) {
+#pragma unroll
+        for (int e = 0; e < VPL; e++) dvw[e] = fma(xo[e], yn[e], dvw[e]);
+      }
+      if (flags & F_AXPY) {
+        T* up = a.u + (int64_t)row * a.ldu + c0;
+        T uo[VPL], un[VPL];
+        uload<T, VPL>(up, uo);
+#pragma unroll
+        for (int e = 0; e < VPL; e++) un[e] = fma(a.gamma, yn[e], a.delta * uo[e]);
+        put_owned<T, VPL>(up, un, own, false);
+      }
+    }
+  }
+
+  if (FULL && (flags & (F_DWW | F_DVW))) {
+    __shared__ T red[2][kBlock / 64][LPR * VPL];
+#pragma unroll
+    for (int e = 0; e < VPL; e++) {
+      dww[e] = wave_sum_strided<LPR>(dww[e]);
+      dvw[e] = wave_sum_strided<LPR>(dvw[e]);
+    }
+    if (lane < LPR) {
+#pragma unroll
+      for (int e = 0; e < VPL; e++)
+        if (e >= own) {
+          red[0][wv][c0 + e] = dww[e];
+          red[1][wv][c0 + e] = dvw[e];
+        }
+    }
+    __syncthreads();
+    const int width = a.ncols;
+    for (int i = threadIdx.x; i < 2 * width; i += kBlock) {
+      const int which = i / width, c = i % width;
+      T s = T(0);
+#pragma unroll
+      for (int k = 0; k < kBlock / 64; k++) s += red[which][k][c];
+      a.partials[(int64_t)blockIdx.x * 2 * width + i] = s;
+    }
+  }
+}
+
+// The products with a Gram epilogue or staged x.
 // One row per LPR lanes; the lanes of a row load the row's val/col
 // cooperatively (lane q takes slot j = jb*LPR + q, coalesced over the rows
 // of the chunk) and share them by group broadcast, so every index is read
@@ -157,9 +367,9 @@ __device__ inline T group_bcast_t(T v, int src, int lane) {
 // registers; the wave tiles are added in LDS in wave order and the
 // workgroup tiles by a second fixed-order pass, so the sums are
 // deterministic.  W itself is not stored with F_NOSTORE (W = NULL).
-template <typename T, int VPL, int LPR, bool XSC, int GR, int SL, bool STG = false>
+template <typename T, int VPL, int LPR, int GR, int SL, bool STG = false>
 __global__ void __launch_bounds__(kBlock) k_sell_spmv(const SpmvArgs<T> a) {
-  static_assert(!STG || (VPL * sizeof(T) >= 16 && !XSC && GR == 0), "staged windows hold whole 16-byte vectors");
+  static_assert(STG ? (VPL * sizeof(T) >= 16 && GR == 0) : GR > 0, "k_spmv takes the plain products");
   constexpr int RPW = 64 / LPR;
   constexpr int RPB = (kBlock / 64) * RPW;
   constexpr int KB = SL > LPR ? SL / LPR : 1;  // val/col loads per lane and batch
@@ -177,11 +387,10 @@ __global__ void __launch_bounds__(kBlock) k_sell_spmv(const SpmvArgs<T> a) {
   const int C = 1 << a.clog2;
   const int flags = a.flags;
 
-  T sh[VPL], xsc[VPL];
+  T sh[VPL];
 #pragma unroll
   for (int e = 0; e < VPL; e++) {
     sh[e] = (colok && (flags & F_SHIFT)) ? (a.shift_dev ? a.shift_dev[c0 + e] : a.shift[c0 + e]) : T(0);
-    if constexpr (XSC) xsc[e] = colok ? (T)a.xscale[(int64_t)(c0 + e) * a.xscale_stride] : T(0);
   }
   T dww[VPL], dvw[VPL];
 #pragma unroll
@@ -371,19 +580,12 @@ __global__ void __launch_bounds__(kBlock) k_sell_spmv(const SpmvArgs<T> a) {
 #pragma unroll
     for (int e = 0; e < VPL; e++) yn[e] = T(0);
     if (live && colok) {
-      if constexpr (XSC) {  // (A + s)(x .* f) = ((A + s) x) .* f, one product per result
-#pragma unroll
-        for (int e = 0; e < VPL; e++) {
-          acc[e] *= xsc[e];
-          xo[e] *= xsc[e];
-        }
-      }
       T* yp = a.y + (int64_t)row * a.ldy + c0;
       if (flags & F_BETA) {
         T yo[VPL];
         vload<T, VPL>(yp, yo);
 #pragma unroll
-        for (int e = 0; e < VPL; e++) yn[e] = a.alpha * acc[e] + a.beta * yo[e];
+        for (int e = 0; e < VPL; e++) yn[e] = fma(a.alpha, acc[e], a.beta * yo[e]);
       } else {
 #pragma unroll
         for (int e = 0; e < VPL; e++) yn[e] = a.alpha * acc[e];
@@ -407,7 +609,7 @@ __global__ void __launch_bounds__(kBlock) k_sell_spmv(const SpmvArgs<T> a) {
         T uo[VPL], un[VPL];
         vload<T, VPL>(up, uo);
 #pragma unroll
-        for (int e = 0; e < VPL; e++) un[e] = a.gamma * yn[e] + a.delta * uo[e];
+        for (int e = 0; e < VPL; e++) un[e] = fma(a.gamma, yn[e], a.delta * uo[e]);
         vstore<T, VPL>(up, un);
       }
     }
@@ -510,14 +712,12 @@ __global__ void __launch_bounds__(kBlock) k_sell_spmv(const SpmvArgs<T> a) {
 
 namespace {
 
-template <typename T, int VPL, int LPR, bool XSC, int GR = 0, int SL = 8, bool STG = false>
-int launch_one(SpmvArgs<T>& a) {
-  auto kern = k_sell_spmv<T, VPL, LPR, XSC, GR, SL, STG>;
-  constexpr int RPB = (kBlock / 64) * (64 / LPR);
-  a.ntiles = (a.nslots + RPB - 1) / RPB;
-  const size_t lds = STG ? a.st_lds_bytes : 0;
+// partial sums of the launch a on `grid` workgroups, then the launch
+template <typename T, typename K>
+int launch_kernel(K kern, SpmvArgs<T>& a, int rows_per_block, size_t lds) {
+  a.ntiles = (a.nslots + rows_per_block - 1) / rows_per_block;
   const int grid = persistent_blocks(kern, lds, a.ntiles, a.blocks_per_cu);
-  if (GR > 0)
+  if (a.flags & (F_GWW | F_GVW))
     a.partials = (T*)device_work(sizeof(T) * (size_t)2 * grid * a.ncols * a.ncols);
   else if (a.flags & (F_DWW | F_DVW))
     a.partials = (T*)device_work(sizeof(T) * ((size_t)grid * 2 * a.ncols + 2 * a.ncols));
@@ -528,51 +728,62 @@ int launch_one(SpmvArgs<T>& a) {
   return grid;
 }
 
-template <typename T, int VPL, bool XSC>
-int launch_lpr(SpmvArgs<T>& a, int lpr) {
-  switch (lpr) {
-    case 1: return launch_one<T, VPL, 1, XSC>(a);
-    case 2: return launch_one<T, VPL, 2, XSC>(a);
-    case 4: return launch_one<T, VPL, 4, XSC>(a);
-    case 8: return launch_one<T, VPL, 8, XSC>(a);
-    case 16: return launch_one<T, VPL, 16, XSC>(a);
-    case 32: return launch_one<T, VPL, 32, XSC>(a);
-    default: return launch_one<T, VPL, 64, XSC>(a);
+// The plain product has an own instance, with fewer registers.  Depth 16 is
+// for it alone: beside the epilogue's registers a batch of 16 leaves too few
+// waves (24-spin chain, 4 columns, shifted: 380 us, 202 at depth 8).
+template <typename T, int VPL, int LPR, int SL>
+int launch_rows(SpmvArgs<T>& a) {
+  constexpr int rows = (kBlock / 64) * (64 / LPR);
+  constexpr int SF = SL == 16 && LPR < 16 ? 8 : SL;
+  if (a.x64) {
+    if constexpr (VPL * sizeof(T) <= 16) return launch_kernel(k_spmv<T, VPL, LPR, SF, true, true>, a, rows, 0);
   }
+  return a.full ? launch_kernel(k_spmv<T, VPL, LPR, SF, true, false>, a, rows, 0)
+                : launch_kernel(k_spmv<T, VPL, LPR, SL, false, false>, a, rows, 0);
 }
-// depth 16 or 32 (rows of many entries; no per-column x factors): row groups of at most 8 lanes
-template <typename T, int VPL, int SL>
-int launch_deep(SpmvArgs<T>& a, int lpr) {
+
+// lanes per row and depth: a batch holds at least one entry per lane, so the
+// wider groups have one depth
+template <typename T, int VPL>
+int launch_vpl(SpmvArgs<T>& a, int lpr, int depth) {
+  if constexpr (VPL * sizeof(T) <= 32) {
+    if (depth >= 16) switch (lpr) {
+        case 1: return launch_rows<T, VPL, 1, 16>(a);
+        case 2: return launch_rows<T, VPL, 2, 16>(a);
+        case 4: return launch_rows<T, VPL, 4, 16>(a);
+        case 8: return launch_rows<T, VPL, 8, 16>(a);
+      }
+  }
+  if (depth <= 4) switch (lpr) {
+      case 1: return launch_rows<T, VPL, 1, 4>(a);
+      case 2: return launch_rows<T, VPL, 2, 4>(a);
+      case 4: return launch_rows<T, VPL, 4, 4>(a);
+    }
   switch (lpr) {
-    case 1: return launch_one<T, VPL, 1, false, 0, SL>(a);
-    case 2: return launch_one<T, VPL, 2, false, 0, SL>(a);
-    case 4: return launch_one<T, VPL, 4, false, 0, SL>(a);
-    default: return launch_one<T, VPL, 8, false, 0, SL>(a);
+    case 1: return launch_rows<T, VPL, 1, 8>(a);
+    case 2: return launch_rows<T, VPL, 2, 8>(a);
+    case 4: return launch_rows<T, VPL, 4, 8>(a);
+    case 8: return launch_rows<T, VPL, 8, 8>(a);
+    case 16: return launch_rows<T, VPL, 16, 16>(a);
+    case 32: return launch_rows<T, VPL, 32, 32>(a);
+    default: return launch_rows<T, VPL, 64, 64>(a);
   }
 }
 
-// the deeper batches hold their gathered values in registers: depth 16 and
-// 32 take at most two 16-byte vectors per lane (wider lanes would need more
-// registers than the file holds without spilling)
-template <typename T, int VPL>
-int launch_xsc(SpmvArgs<T>& a, int lpr, int depth) {
-  if (!a.xscale && lpr <= 8) {
-    if constexpr (VPL * sizeof(T) <= 32)
-      if (depth >= 32) return launch_deep<T, VPL, 32>(a, lpr);
-    if constexpr (VPL * sizeof(T) <= 32)
-      if (depth >= 16) return launch_deep<T, VPL, 16>(a, lpr);
-  }
-  return a.xscale ? launch_lpr<T, VPL, true>(a, lpr) : launch_lpr<T, VPL, false>(a, lpr);
+template <typename T, int VPL, int LPR, int GR, int SL, bool STG>
+int launch_one(SpmvArgs<T>& a) {
+  return launch_kernel(k_sell_spmv<T, VPL, LPR, GR, SL, STG>, a, (kBlock / 64) * (64 / LPR),
+                       STG ? a.st_lds_bytes : 0);
 }
 
 // staged windows (row groups of at most 8 lanes of 16-byte vectors): depth 8, or 16 for lanes of at most 32 bytes
 template <typename T, int VPL, int SL>
 int launch_stage_sl(SpmvArgs<T>& a, int lpr) {
   switch (lpr) {
-    case 1: return launch_one<T, VPL, 1, false, 0, SL, true>(a);
-    case 2: return launch_one<T, VPL, 2, false, 0, SL, true>(a);
-    case 4: return launch_one<T, VPL, 4, false, 0, SL, true>(a);
-    default: return launch_one<T, VPL, 8, false, 0, SL, true>(a);
+    case 1: return launch_one<T, VPL, 1, 0, SL, true>(a);
+    case 2: return launch_one<T, VPL, 2, 0, SL, true>(a);
+    case 4: return launch_one<T, VPL, 4, 0, SL, true>(a);
+    default: return launch_one<T, VPL, 8, 0, SL, true>(a);
   }
 }
 template <typename T, int VPL>
@@ -586,12 +797,12 @@ int launch_stage(SpmvArgs<T>& a, int lpr, int depth) {
 template <typename T, int VPL, int GR>
 int launch_gram_lpr(SpmvArgs<T>& a, int lpr) {
   switch (lpr) {
-    case 1: return launch_one<T, VPL, 1, false, GR>(a);
-    case 2: return launch_one<T, VPL, 2, false, GR>(a);
-    case 4: return launch_one<T, VPL, 4, false, GR>(a);
-    case 8: return launch_one<T, VPL, 8, false, GR>(a);
-    case 16: return launch_one<T, VPL, 16, false, GR>(a);
-    default: return launch_one<T, VPL, 32, false, GR>(a);
+    case 1: return launch_one<T, VPL, 1, GR, 8, false>(a);
+    case 2: return launch_one<T, VPL, 2, GR, 8, false>(a);
+    case 4: return launch_one<T, VPL, 4, GR, 8, false>(a);
+    case 8: return launch_one<T, VPL, 8, GR, 8, false>(a);
+    case 16: return launch_one<T, VPL, 16, GR, 8, false>(a);
+    default: return launch_one<T, VPL, 32, GR, 8, false>(a);
   }
 }
 template <typename T, int VPL>
@@ -606,6 +817,18 @@ __global__ void __launch_bounds__(kBlock) k_spmv_gram_out(const T* __restrict__ 
   const T s = block_sum16(partials, nblocks, n * n);
   const int o = blockIdx.x * 16 + threadIdx.x;
   if (threadIdx.x < 16 && o < n * n) C[(int64_t)(o / n) * ldc + o % n] = s;
+}
+
+// the sums of k_reduce_partials over [nblocks][2][n] partials: the first n to
+// ww, the others to vw (either may be null)
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_spmv_dots_out(const T* __restrict__ partials, int nblocks, int n, T* ww,
+                                                          T* vw) {
+  const T s = block_sum16(partials, nblocks, 2 * n);
+  const int o = blockIdx.x * 16 + threadIdx.x;
+  if (threadIdx.x >= 16 || o >= 2 * n) return;
+  T* out = o < n ? ww : vw;
+  if (out) out[o < n ? o : o - n] = s;
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -635,6 +858,68 @@ const SellStage* spmv_stage_for(const SparseMat<T>* A, int nc, int vpl, int* psh
 template const SellStage* spmv_stage_for<double>(const SparseMat<double>*, int, int, int*, size_t*);
 template const SellStage* spmv_stage_for<float>(const SparseMat<float>*, int, int, int*, size_t*);
 
+// rows whose products always take the instance with epilogues: it keeps
+// fewer gathers under way per wave, which long rows want (their x lines miss
+// the L1, and more lines under way than it holds evict each other; 4.2 M rows
+// x 32 in a band of +-50k, us: 8 columns 1001 against 1157, 4 columns 703 /
+// 815, 16: 1622 / 1805; 300 k x 24 in +-400, 8 columns 44 / 48)
+template <typename T>
+inline bool spmv_long_rows(const SparseMat<T>* A) {
+  return A->nnz >= 24 * std::max<int64_t>(1, A->nrows);
+}
+
+// Launch of k_spmv for a matrix without settings, from sweeps over lane
+// widths, depths, workgroups per CU and column blocks (us; "b" = workgroups
+// per CU; plain / shifted = the two instances):
+//  - long rows: depth 8; x rows of 128 bytes and more in 32-byte lanes (16
+//    columns 1622 against 1987 and more), wider blocks in launches of 128
+//    bytes (32 columns: 3280 against 4550); where the columns of neighbouring
+//    rows span more of x than a share of the L2 (512 KB), narrow x rows want
+//    few workgroups (+-50k, 1 column: 788 at b1, 880 from b3; 4 columns: 703
+//    at b3, 790 from b4)
+//  - rows of 9 to 23 entries, plain: depth 16 (24-spin chain, 4 columns: FP64
+//    177 against 191 at depth 8, FP32 106 / 112; graphene, 8 columns 80 /
+//    80), 32-byte lanes for x rows of 128 bytes (16 columns: 528 against
+//    600); shifted: depth 8, x rows of 32 bytes gathered over a wide span in
+//    one lane (chain, 4 columns: 190 at b2, 256 in two lanes; 1 M x 12 in
+//    +-3000: 93 in one, 70 in two), from 128 bytes on b4 (601 / 629)
+//  - rows of at most 8 entries (a 3D stencil): one batch; x rows of 32 bytes
+//    in one lane (64 x 58 x 51 grid: 5.9 against 6.8, 128^3 shifted: 66 /
+//    79), from 64 bytes on b4 (128^3, 8 columns: 106 at b4, 111 at b6; 16:
+//    213 / 219), shifted only from 128 (8 columns 143 at b4, 125 at b6)
+//  - rows of at most 4 entries (a sheet): x rows of 128 bytes and more in
+//    32-byte lanes, b3 (8 M rows, 32 columns: 1092 against 1470 in 16-byte
+//    lanes; 12 columns, 96 bytes: 466 / 475), else b6 (5 columns: 45 at b6,
+//    55 at b4)
+template <typename T>
+SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
+  SpmvTuned d;
+  const int rb = nvec * (int)sizeof(T);
+  d.blocks_per_cu = 0;
+  const bool wide = 4.0 * A->gather_span * rb >= 512.0 * 1024.0;  // the span of x that neighbouring rows read
+  if (spmv_long_rows(A)) {
+    if (rb > 128) d.col_block = 128 / (int)sizeof(T);
+    d.lane_bytes = rb >= 128 ? 32 : 0;
+    if (wide && rb <= 32) d.blocks_per_cu = rb <= 8 ? 1 : 3;
+  } else if (A->max_row_len > 8) {
+    if (full) {
+      const bool far = rb == 32 && wide;
+      d.lane_bytes = far ? 32 : 0;
+      d.blocks_per_cu = far ? 2 : rb >= 128 ? 4 : 0;
+    } else {
+      d.depth = rb > 8 ? 16 : 8;
+      d.lane_bytes = rb >= 128 ? 32 : 0;
+    }
+  } else if (A->max_row_len > 4) {
+    d.lane_bytes = rb == 32 || rb >= 256 ? 32 : 0;
+    d.blocks_per_cu = rb >= (full ? 128 : 64) ? 4 : 6;
+  } else {
+    d.lane_bytes = rb >= 128 ? 32 : 0;
+    d.blocks_per_cu = rb >= 128 ? 3 : 6;
+  }
+  return d;
+}
+
 template <typename T>
 void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mvec<T>* x, T beta, Mvec<T>* y,
                  const SpmvRequest& req, T* dot_ww_host, T* dot_vw_host, T gamma, T delta, Mvec<T>* U) {
@@ -661,44 +946,59 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
                 "x and y overlap in memory");
 
   constexpr int V16 = 16 / sizeof(T);
+  // whole 16-byte vectors in every row: what the staged and Gram kernels need
   bool vec_ok = (nvec % V16 == 0) && (x->lda % V16 == 0) && aligned16(x->dev());
   if (y) vec_ok = vec_ok && (y->lda % V16 == 0) && aligned16(y->dev());
   if (req.axpy_u) vec_ok = vec_ok && (U->lda % V16 == 0) && aligned16(U->dev());
-  int VPL = vec_ok ? V16 : 1;
-  const auto tuned = A->tuned.find(nvec);
-  if (!gram) {  // the gathered bytes per lane and nonzero (same sums whichever is taken)
-    int lb = rt().spmv_lane_bytes;
-    if (req.lane_bytes >= 0)
-      lb = req.lane_bytes;
-    else if (lb == 0 && tuned != A->tuned.end())
-      lb = tuned->second.lane_bytes;
-    const int w = lb / (int)sizeof(T);
-    if (lb > 0 && lb <= (int)sizeof(T)) {
-      VPL = 1;
-    } else if (vec_ok && (w == 2 * V16 || w == 4 * V16)) {
-      bool ok = nvec % w == 0 && x->lda % w == 0;
-      if (y) ok = ok && y->lda % w == 0;
-      if (req.axpy_u) ok = ok && U->lda % w == 0;
-      if (ok) VPL = w;
-    }
+  const auto tuned_at = A->tuned.find(nvec);
+  const bool full = spmv_long_rows(A) || req.has_shift || req.has_beta || req.dot_ww || req.dot_vw || req.axpy_u ||
+                    req.xscale;
+  const SpmvTuned preset = tuned_at != A->tuned.end() ? tuned_at->second : spmv_default_launch(A, nvec, full);
+  // x rows of each tile staged in LDS (where the matrix's tiles allow it)
+  int stage = req.stage;
+  if (stage < 0) stage = rt().spmv_stage;
+  if (stage < 0) stage = preset.stage;
+  // block columns per lane, the gathered bytes per lane and nonzero, and per
+  // launch: 64 lane groups, or fewer as set or tuned (each further launch
+  // reads the matrix again); each row's sum is the same whichever is taken.
+  // x rows are addressed by 32-bit byte offsets from the block's first row;
+  // larger blocks (x64) take one vector per lane.
+  const bool x64 = !gram && (uint64_t)x->nrows * (uint64_t)x->lda * sizeof(T) > UINT32_MAX;
+  const bool tuned = tuned_at != A->tuned.end();
+  int VPL = 1, maxcols = 64;
+  auto shape = [&](bool with_preset) {
+    int lb = rt().spmv_lane_bytes, colblock = req.col_block;
+    if (req.lane_bytes >= 0) lb = req.lane_bytes;
+    else if (lb == 0 && with_preset) lb = preset.lane_bytes;
+    if (colblock < 0) colblock = rt().spmv_col_block;
+    if (colblock < 0) colblock = with_preset ? preset.col_block : 0;
+    VPL = spmv_lane_columns<T>(nvec, x64 && lb > 16 ? 0 : lb);
+    maxcols = 64 * VPL;
+    if (colblock > 0 && colblock % VPL == 0) maxcols = std::min(maxcols, colblock);
+  };
+  bool staged = false;
+  if (gram) {
+    VPL = vec_ok ? V16 : 1;
+    maxcols = 64 * VPL;
+  } else {
+    // staging forced on or off keeps the 16-byte lanes either way, so that both products' dots group alike
+    shape(tuned || (req.stage < 0 && rt().spmv_stage < 0));
+    if (stage > 0 && vec_ok && !req.xscale)
+      staged = spmv_stage_for(A, std::min(nvec, maxcols), VPL, nullptr, nullptr) != nullptr;
   }
-  // block columns per launch: 64 lane groups, or fewer as set or tuned (each
-  // further launch reads the matrix again; each row's sum is the same)
-  int maxcols = 64 * VPL;
-  int colblock = req.col_block;
-  if (colblock < 0) colblock = rt().spmv_col_block;
-  if (colblock < 0) colblock = tuned != A->tuned.end() ? tuned->second.col_block : 0;
-  if (!gram && colblock > 0 && colblock % VPL == 0) maxcols = std::min(maxcols, colblock);
 
   SpmvArgs<T> a;
   a.chunk_ptr = A->d_chunk_ptr;
   a.chunk_w = A->d_chunk_w;
-  a.perm = A->d_perm;
+  a.perm = A->perm_identity && !gram ? nullptr : A->d_perm;
   a.col = A->d_col;
   a.val = A->d_val;
   int clog2 = 0;
   while ((1 << clog2) < A->C) clog2++;
   a.clog2 = clog2;
+  a.nrows = A->nrows;
+  a.x64 = x64;
+  a.full = full;
   a.nslots = A->nchunks * A->C;
   a.ldx = x->lda;
   a.ldy = y ? y->lda : 0;
@@ -713,29 +1013,17 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   if (y && (rt().spmv_nt_y == 1 || (rt().spmv_nt_y < 0 && (int64_t)sizeof(T) * y->nrows * nvec >= Runtime::kNtYBytes &&
                                      (int)sizeof(T) * nvec < 128)))
     a.flags |= F_NTY;
-  if (req.blocks_per_cu >= 0)
-    a.blocks_per_cu = req.blocks_per_cu;
-  else if (rt().spmv_blocks_per_cu >= 0)
-    a.blocks_per_cu = rt().spmv_blocks_per_cu;
-  else if (tuned != A->tuned.end())
-    a.blocks_per_cu = tuned->second.blocks_per_cu;
-  else
-    a.blocks_per_cu = spmv_table_blocks_per_cu(A->nrows ? (double)A->nnz / (double)A->nrows : 0.0, nvec);
-  // entries per row whose loads go out together (8 or 32)
-  int depth;
-  if (req.depth >= 0)
-    depth = req.depth;
-  else if (rt().spmv_depth >= 0)
-    depth = rt().spmv_depth;
-  else if (tuned != A->tuned.end())
-    depth = tuned->second.depth;
-  else
-    depth = 8;
+  // workgroups per CU
+  int bpc = req.blocks_per_cu;
+  if (bpc < 0) bpc = rt().spmv_blocks_per_cu;
+  const bool bpc_set = bpc >= 0 || tuned;
+  a.blocks_per_cu = bpc >= 0 ? bpc : preset.blocks_per_cu;
+  // entries per row whose loads go out together
+  int depth = req.depth;
+  if (depth < 0) depth = rt().spmv_depth;
+  if (depth < 0) depth = preset.depth;
+  if (A->max_row_len <= 4) depth = std::min(depth, 4);  // a batch beyond the longest row only costs registers
   const bool dots = req.dot_ww || req.dot_vw;
-  // x rows of each tile staged in LDS (where the matrix's tiles allow it)
-  int stage = req.stage;
-  if (stage < 0) stage = rt().spmv_stage;
-  if (stage < 0) stage = tuned != A->tuned.end() ? tuned->second.stage : 0;
   a.st_ivptr = nullptr;
   a.st_iv = nullptr;
   a.st_lcol = nullptr;
@@ -751,13 +1039,19 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
     a.u = U ? U->dev() + cb : nullptr;
     a.shift_dev = (req.has_shift && req.shifts_dev) ? static_cast<const T*>(req.shifts_dev) + cb : nullptr;
     for (int c = 0; c < nc; c++) a.shift[c] = (req.has_shift && !a.shift_dev) ? shifts_host[cb + c] : T(0);
-    const int groups = (nc + VPL - 1) / VPL;
+    int vpl = VPL;
+    while (vpl > nc) vpl /= 2;  // the last columns of a wide block
+    const int groups = (nc + vpl - 1) / vpl;
     int lpr = 1;
     while (lpr < groups) lpr <<= 1;
     a.xscale = req.xscale ? req.xscale + (int64_t)cb * req.xscale_stride : nullptr;
     a.xscale_stride = req.xscale_stride;
+    const int staged_bpc =
+        bpc_set ? a.blocks_per_cu
+                : spmv_table_blocks_per_cu(A->nrows ? (double)A->nnz / (double)A->nrows : 0.0, nvec);
     if (gram) {  // one column block (nvec <= 32)
-      const int grid = VPL == 1 ? launch_gram<T, 1>(a, lpr) : launch_gram<T, V16>(a, lpr);
+      a.blocks_per_cu = staged_bpc;
+      const int grid = vec_ok ? launch_gram<T, V16>(a, lpr) : launch_gram<T, 1>(a, lpr);
       const int nn = nc * nc;
       if (req.gram_ww_dev) {
         hipLaunchKernelGGL(k_spmv_gram_out<T>, dim3((nn + 15) / 16), dim3(kBlock), 0, rt().stream, a.partials, grid,
@@ -772,39 +1066,40 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
       }
       continue;
     }
-    const SellStage* S = stage > 0 && !a.xscale ? spmv_stage_for(A, nc, VPL, &a.st_pshift, &a.st_lds_bytes) : nullptr;
+    const SellStage* S = staged && vpl % V16 == 0 && nc % vpl == 0
+                             ? spmv_stage_for(A, nc, vpl, &a.st_pshift, &a.st_lds_bytes)
+                             : nullptr;
     int grid;
     if (S) {
       rt().spmv_staged_launches++;
+      a.blocks_per_cu = staged_bpc;
+      a.perm = A->d_perm;
       a.st_ivptr = S->d_ivptr;
       a.st_iv = S->d_iv;
       a.st_lcol = S->d_lcol;
       a.st_ppr = nc * (int)sizeof(T) / 16;
-      grid = VPL == V16 ? launch_stage<T, V16>(a, lpr, depth)
-                        : (VPL == 2 * V16 ? launch_stage<T, 2 * V16>(a, lpr, depth) : launch_stage<T, 4 * V16>(a, lpr, depth));
+      grid = vpl == V16 ? launch_stage<T, V16>(a, lpr, depth)
+                        : (vpl == 2 * V16 ? launch_stage<T, 2 * V16>(a, lpr, depth) : launch_stage<T, 4 * V16>(a, lpr, depth));
     } else {
-      grid = VPL == 1     ? launch_xsc<T, 1>(a, lpr, depth)
-             : VPL == V16 ? launch_xsc<T, V16>(a, lpr, depth)
-             : VPL == 2 * V16 ? launch_xsc<T, 2 * V16>(a, lpr, depth)
-                              : launch_xsc<T, 4 * V16>(a, lpr, depth);
+      switch (vpl) {
+        case 1: grid = launch_vpl<T, 1>(a, lpr, depth); break;
+        case 2: grid = launch_vpl<T, 2>(a, lpr, depth); break;
+        case 4: grid = launch_vpl<T, 4>(a, lpr, depth); break;
+        case 8: grid = launch_vpl<T, 8>(a, lpr, depth); break;
+        default: grid = launch_vpl<T, 4 * V16>(a, lpr, depth); break;
+      }
     }
     if (dots && req.dots_dev && cb == 0 && nc == nvec) {
       hipLaunchKernelGGL(k_reduce_partials<T>, dim3((2 * nc + 15) / 16), dim3(kBlock), 0, rt().stream, a.partials,
                          grid, 2 * nc, static_cast<T*>(req.dots_dev));
       PHX_HIP(hipGetLastError());
     } else if (dots && (req.dots_dev || req.dot_ww_dev || req.dot_vw_dev)) {
-      // fixed-order sums into the tail of the partials buffer (sized for them), then to the two outputs
-      // (dots_dev: ww at [0, nvec), vw at [nvec, 2 nvec), this block's columns at offset cb)
-      T* sums = a.partials + (size_t)grid * 2 * nc;
-      hipLaunchKernelGGL(k_reduce_partials<T>, dim3((2 * nc + 15) / 16), dim3(kBlock), 0, rt().stream, a.partials,
-                         grid, 2 * nc, sums);
-      PHX_HIP(hipGetLastError());
+      // dots_dev: ww at [0, nvec), vw at [nvec, 2 nvec), this block's columns at offset cb
       T* ww_out = req.dots_dev ? static_cast<T*>(req.dots_dev) : static_cast<T*>(req.dot_ww_dev);
       T* vw_out = req.dots_dev ? static_cast<T*>(req.dots_dev) + nvec : static_cast<T*>(req.dot_vw_dev);
-      if (ww_out)
-        PHX_HIP(hipMemcpyAsync(ww_out + cb, sums, sizeof(T) * nc, hipMemcpyDeviceToDevice, rt().stream));
-      if (vw_out)
-        PHX_HIP(hipMemcpyAsync(vw_out + cb, sums + nc, sizeof(T) * nc, hipMemcpyDeviceToDevice, rt().stream));
+      hipLaunchKernelGGL(k_spmv_dots_out<T>, dim3((2 * nc + 15) / 16), dim3(kBlock), 0, rt().stream, a.partials, grid,
+                         nc, ww_out ? ww_out + cb : nullptr, vw_out ? vw_out + cb : nullptr);
+      PHX_HIP(hipGetLastError());
     } else if (dots) {
       std::vector<T> sums(2 * nc);
       reduce_partials_to_host(a.partials, grid, 2 * nc, sums.data());

@@ -10,9 +10,8 @@
 //   * per block width, the workgroups per CU of the persistent grid (the
 //     number of waves in flight, which trades latency hiding against the L2
 //     footprint of the gathered x rows);
-//   * per block width, for rows of at least 16 entries, the depth: 8, 16 or
-//     32 entries of a row whose index loads and gathers go out together (16
-//     and 32 also prefetch the next batch's indices);
+//   * per block width, for rows of 9 to 23 entries, the depth: 8 or 16
+//     entries of a row whose index loads and gathers go out together;
 //   * per block width above 16 columns, launches of 16 (and above 32, of 32)
 //     columns instead of one: each reads the matrix again, but gathers rows
 //     of x half (a quarter) as wide, so fewer of them leave L2;
@@ -126,19 +125,6 @@ double time_product(const SparseMat<T>* A, Mvec<T>* x, Mvec<T>* y, int lb, int b
   return best;
 }
 
-// the scalars per lane the SpMV takes for a block of nvec contiguous columns
-// (lda = nvec, 16-byte aligned) and lane_bytes lb; candidates that give the
-// same kernel are tried once
-template <typename T>
-int lanes_vpl(int nvec, int lb) {
-  constexpr int V16 = 16 / sizeof(T);
-  const bool vec_ok = nvec % V16 == 0;
-  if (lb > 0 && lb <= (int)sizeof(T)) return 1;
-  const int w = lb / (int)sizeof(T);
-  if (vec_ok && (w == 2 * V16 || w == 4 * V16) && nvec % w == 0) return w;
-  return vec_ok ? V16 : 1;
-}
-
 template <typename T>
 SpmvTuned search_launch(const SparseMat<T>* A, int nvec, int reps) {
   TrialBlock<T> x(A->col_map, A->ncols, nvec), y(A->row_map, A->nrows, nvec);
@@ -146,8 +132,7 @@ SpmvTuned search_launch(const SparseMat<T>* A, int nvec, int reps) {
   best.ms = 1e300;
   std::vector<int> seen;
   std::vector<int> depths{8};
-  if (A->max_row_len >= 16) depths.push_back(16);
-  if (A->max_row_len >= 24) depths.push_back(32);
+  if (A->max_row_len > 8 && A->nnz < 24 * A->nrows) depths.push_back(16);  // (long rows run depth 8)
   std::vector<int> blocks{0};
   for (int w : {16, 32})
     if (nvec > w) blocks.push_back(w);
@@ -155,7 +140,7 @@ SpmvTuned search_launch(const SparseMat<T>* A, int nvec, int reps) {
     seen.clear();
     const int ncol = cbw > 0 ? cbw : nvec;  // the widest launch
     for (int lb : {0, (int)sizeof(T), 32, 64}) {
-      const int vpl = lanes_vpl<T>(nvec, lb);
+      const int vpl = spmv_lane_columns<T>(nvec, lb);  // candidates that give the same kernel are tried once
       if (std::find(seen.begin(), seen.end(), vpl) != seen.end()) continue;
       seen.push_back(vpl);
       if (cbw > 0 && cbw % vpl != 0) continue;

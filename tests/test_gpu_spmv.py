@@ -501,3 +501,84 @@ def test_spmv_lane_widths_bitexact(be64, be32, dtype, nvec):
     for o in (x, A):
         o.delete()
     m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["sheet", "stencil", "band12", "band30"])
+def test_spmv_widths_by_column(be64, be32, kind, dtype):
+    """every block width runs each column's own sum: the columns of a block
+    product equal the one-column products bit for bit, whole vectors and
+    ragged widths, rows of at most 4, of 7, 12 and 30 entries, plain and
+    shifted with beta, on whole blocks and on a column view that starts and
+    ends unaligned; the columns next to the view stay as they were; the dots
+    agree with the columns"""
+    be = be64 if dtype == np.float64 else be32
+    A = {"sheet": lambda: be.honeycomb(37, 23, 0, 0, 0, 1.0, 7), "stencil": lambda: be.laplace3d(13, 7, 9),
+         "band12": lambda: be.banded_random(1001, 12, 60, 40.0, 5),
+         "band30": lambda: be.banded_random(997, 30, 400, 40.0, 6)}[kind]()
+    n, widest = A.nrows, 133
+    rng = np.random.default_rng(17)
+    X, Y0 = (rng.uniform(-1, 1, (n, widest)).astype(dtype) for _ in range(2))
+    sh = rng.uniform(-2, 2, widest).astype(dtype)
+    m = be.map(n)
+    one, shifted = np.empty_like(X), np.empty_like(X)
+    x, y = be.mvec(m, 1), be.mvec(m, 1)
+    for c in range(widest):
+        x.set(X[:, c:c + 1])
+        be.spmv(0.75, A, x, 0.0, y)
+        one[:, c:c + 1] = y.get()
+        y.set(Y0[:, c:c + 1])
+        be.spmv_shifted(0.75, A, sh[c:c + 1], x, -0.3, y)
+        shifted[:, c:c + 1] = y.get()
+    x.delete()
+    y.delete()
+    tol = 1e-12 if dtype == np.float64 else 1e-4  # sums of at most 1001 terms, products of like sign summed
+    for k in (2, 3, 4, 5, 6, 7, 8, 9, 12, 15, 16, 17, 31, 32, 33, 63, 65, 129, 133):
+        x, y = be.mvec(m, k, X[:, :k]), be.mvec(m, k, Y0[:, :k])
+        be.spmv(0.75, A, x, 0.0, y)
+        assert np.array_equal(y.get(), one[:, :k]), k
+        y.set(Y0[:, :k])
+        be.spmv_shifted(0.75, A, sh[:k], x, -0.3, y)
+        assert np.array_equal(y.get(), shifted[:, :k]), k
+        if k <= 64:
+            ww, vw = be.fused_spmv_mvdot(0.75, A, x, 0.0, y)
+            assert np.array_equal(y.get(), one[:, :k]), k
+            w, v = one[:, :k].astype(float), X[:, :k].astype(float)
+            assert np.all(np.abs(ww - (w * w).sum(0)) <= tol * (w * w).sum(0)), k
+            assert np.all(np.abs(vw - (v * w).sum(0)) <= tol * np.abs(v * w).sum(0)), k
+        x.delete()
+        y.delete()
+        big = np.full((n, k + 2), 3.0, dtype)
+        big[:, 1:k + 1] = X[:, :k]
+        X2, Y2 = be.mvec(m, k + 2, big), be.mvec(m, k + 2, np.full((n, k + 2), 5.0, dtype))
+        x, y = X2.view(1, k), Y2.view(1, k)
+        be.spmv(0.75, A, x, 0.0, y)
+        got = Y2.get()
+        assert np.array_equal(got[:, 1:k + 1], one[:, :k]), k
+        assert np.all(got[:, [0, k + 1]] == 5.0), k
+        for o in (x, y, X2, Y2):
+            o.delete()
+    A.delete()
+    m.delete()
+
+
+@pytest.mark.parametrize("k", [1, 3, 4])
+def test_spmv_block_over_4_gib(be64, k):
+    """x rows beyond 4 GiB of their block (a view of a wide block, 64-bit
+    offsets): the product of the compact block, bit for bit"""
+    A = be64.laplace3d(108, 107, 106)
+    n, ld = A.nrows, 448
+    assert n * ld * 8 > 2**32
+    m = be64.map(n)
+    X = np.random.default_rng(3).uniform(-1, 1, (n, k))
+    x, y = be64.mvec(m, k, X), be64.mvec(m, k)
+    be64.spmv(1.0, A, x, 0.0, y)
+    want = y.get()
+    wide = be64.mvec(m, ld)
+    xv = wide.view(ld - k, ld - 1)
+    be64.call("mvec_add_mvec", be64.s(1.0), x.h, be64.s(0.0), xv.h)
+    be64.spmv(1.0, A, xv, 0.0, y)
+    assert np.array_equal(y.get(), want)
+    for o in (xv, wide, x, y, A):
+        o.delete()
+    m.delete()
