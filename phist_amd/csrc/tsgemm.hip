@@ -169,7 +169,8 @@ struct Mfma<float> {
   __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
-// S = a'b for na, nb <= 32 (TM = ceil(na/16), TK = ceil(nb/16)); a wave
+// S = a'b for na, nb <= 32, or na <= 64 and nb <= 16 (TM = ceil(na/16), TK =
+// ceil(nb/16)); a wave
 // consumes 16 rows per tile (four 4-row MFMA steps), two tiles per
 // iteration so that both tiles' loads are in flight together; with SELF
 // (a == b) only the upper block tiles are computed and mirrored.  With PAIR
@@ -454,12 +455,16 @@ static bool gram_self_sets(T alpha, const T* a, int64_t lda, int k, int64_t nrow
   return true;
 }
 
-// S = a'b on the matrix cores for na, nb <= 32 (zero-padded to 16-column
-// tiles), written to C as C = alpha*S + beta*C; Cmirror, when given,
-// receives the transposed block from the same partial sums
+// S = a'b on the matrix cores for na, nb <= 32, or na <= 64 and nb <= 16
+// (zero-padded to 16-column tiles), written to C as C = alpha*S + beta*C, or
+// its transpose; Cmirror, when given, receives the transposed block from the
+// same partial sums.  A wide a against a narrow b is one pass over both: two
+// passes of 32 columns read b and the lines at the seam twice and leave the
+// second pass half empty (2.7 M rows, 40 x 4 columns, FP64: 255 us in
+// launches of 32 and 8 columns, 192 us in one, 4.9 TB/s).
 template <typename T>
 static void gram_block_mfma(T alpha, const T* a, int64_t lda, int na, const T* b, int64_t ldb, int nb, int64_t nrows,
-                            bool self, T beta, T* Cdev, int ldc, T* Cmirror = nullptr) {
+                            bool self, T beta, T* Cdev, int ldc, T* Cmirror = nullptr, bool transposed = false) {
   GramArgs<T> g;
   g.nrows = nrows;
   g.a = a;
@@ -478,13 +483,15 @@ static void gram_block_mfma(T alpha, const T* a, int64_t lda, int na, const T* b
   else if (self) nparts = gram_mfma_launch<T, 2, 2, true>(g);
   else if (tm == 1 && tk == 1) nparts = gram_mfma_launch<T, 1, 1, false>(g);
   else if (tm == 1) nparts = gram_mfma_launch<T, 1, 2, false>(g);
-  else if (tk == 1) nparts = gram_mfma_launch<T, 2, 1, false>(g);
+  else if (tk == 1 && tm == 2) nparts = gram_mfma_launch<T, 2, 1, false>(g);
+  else if (tk == 1 && tm == 3) nparts = gram_mfma_launch<T, 3, 1, false>(g);
+  else if (tk == 1) nparts = gram_mfma_launch<T, 4, 1, false>(g);
   else if (pair) nparts = gram_mfma_launch<T, 2, 2, false, true>(g);
   else nparts = gram_mfma_launch<T, 2, 2, false>(g);
   const int nout = na * nb;
   const int fblocks = finalize_blocks(nout);
   hipLaunchKernelGGL(k_gram_finalize<T>, dim3(fblocks), dim3(kBlock), 0, rt().stream, g.partials, nparts, na, nb,
-                     false, alpha, beta, Cdev, ldc);
+                     transposed, alpha, beta, Cdev, ldc);
   PHX_HIP(hipGetLastError());
   if (Cmirror) {  // the transposed block of a self Gram, from the same partials
     hipLaunchKernelGGL(k_gram_finalize<T>, dim3(fblocks), dim3(kBlock), 0, rt().stream, g.partials, nparts, na, nb,
@@ -552,8 +559,19 @@ void gemm_gram(T alpha, const Mvec<T>* V, const Mvec<T>* W, T beta, SdMat<T>* C,
     return;
   }
   if (rt().gram_mfma && (wide >= rt().gram_mfma_wide || (strided && wide >= 4) || (self && wide >= 8))) {
-    // matrix cores: 32 x 32 output blocks (the self Gram computes the upper
+    // matrix cores: a narrow side of at most 16 columns takes 64 of the other
+    // at a time, else 32 x 32 output blocks (the self Gram computes the upper
     // blocks and mirrors them)
+    if (!self && std::min(m, k) <= 16 && wide > 32) {
+      const bool tr = k > m;  // the wide side is sliced
+      const Mvec<T>* A = tr ? W : V;
+      const Mvec<T>* B = tr ? V : W;
+      for (int i0 = 0; i0 < wide; i0 += 64)
+        gram_block_mfma<T>(alpha, A->dev() + i0, A->lda, std::min(64, wide - i0), B->dev(), B->lda, B->nvec, V->nrows,
+                           false, beta, tr ? C->dev() + (int64_t)i0 * ldc : C->dev() + i0, ldc, nullptr, tr);
+      if (to_host) sd_from_device(C);
+      return;
+    }
     for (int i0 = 0; i0 < m; i0 += 32)
       for (int j0 = 0; j0 < k; j0 += 32) {
         const int mi = std::min(32, m - i0), kj = std::min(32, k - j0);
@@ -736,8 +754,9 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
   // are disjoint and each row's stores follow its own loads)
   constexpr int UNR = (GRAM == 0 && KS * TM <= 16) ? 2 : 1;
   const TileWalk tw = xcd_tiles(p.ntiles);
+  const bool upd = p.mode == 0 && p.beta != T(0);  // W's old values, requested with V's
   for (int64_t t0 = tw.t; t0 < tw.end; t0 += UNR * tw.stride) {
-  T au[UNR][RT][KS];
+  T au[UNR][RT][KS], wold[UNR][RT][TM][4];
 #pragma unroll
   for (int u = 0; u < UNR; u++) {
     const int64_t tu = t0 + u * tw.stride;
@@ -761,6 +780,18 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
 #pragma unroll
         for (int st = 0; st < KS; st++) au[u][rt_][st] = (tok && ra < p.nrows && j0 + st < p.k) ? vp[st] : T(0);
       }
+    }
+    if (upd) {
+#pragma unroll
+      for (int rt_ = 0; rt_ < RT; rt_++)
+#pragma unroll
+        for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const int64_t row = r0 + rt_ * 16 + M::row(lane, r);
+            const int c = tm * 16 + cc;
+            wold[u][rt_][tm][r] = (tok && row < p.nrows && c < p.m) ? p.w[row * p.ldw + c] : T(0);
+          }
     }
   }
 #pragma unroll
@@ -789,7 +820,7 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
           if (row < p.nrows && c < p.m) {
             T* wp = p.w + row * p.ldw + c;
             T val = acc[rt_][tm][r];
-            if (p.mode == 0 && p.beta != T(0)) val = fma(p.beta, *wp, val);
+            if (upd) val = fma(p.beta, wold[u][rt_][tm][r], val);
             *wp = val;
             acc[rt_][tm][r] = val;  // the Gram epilogue uses the stored values
           }
@@ -933,13 +964,32 @@ bool mix_mfma_ok(int mode, int k, int m) {
   return rt().mix_mfma && mode != 1 && k >= 8 && m >= rt().mix_mfma_min_m && k <= 64 && m <= 64;
 }
 
+// columns of V per lane group: a quarter of k, rounded up so that the groups
+// start on whole vectors; with fewer sizes the last groups run half empty and
+// the one at the end of the row falls back to scalar loads (2.7 M rows, FP64:
+// W -= V C of 40 -> 4 columns 301 us with 16 per group, 217 us with 10, 4.8
+// TB/s).  Outputs wider than 16 columns keep groups of whole 128-byte lines:
+// there the spare group costs less than its split lines (48 -> 24 columns:
+// 297 us with 16 per group, 317 us with 12).
+template <typename T>
+int mix_group(int k, int m) {
+  const int ks = (k + 3) / 4;
+  if (m > 16) return ks <= 2 ? 2 : ks <= 4 ? 4 : ks <= 8 ? 8 : 16;
+  if (sizeof(T) == 8 && ks > 4 && ks <= 6) return 6;
+  if (sizeof(T) == 8 && ks > 8 && ks <= 10) return 10;
+  return ks <= 2 ? 2 : ks <= 4 ? 4 : ks <= 8 ? 8 : ks <= 12 ? 12 : 16;
+}
+
 template <typename T>
 void mix_mfma(MixArgs<T>& p) {
-  const int ks = (p.k + 3) / 4;
-  if (ks <= 2) mix_mfma_tm<T, 2>(p);
-  else if (ks <= 4) mix_mfma_tm<T, 4>(p);
-  else if (ks <= 8) mix_mfma_tm<T, 8>(p);
-  else mix_mfma_tm<T, 16>(p);
+  switch (mix_group<T>(p.k, p.m)) {
+    case 2: return mix_mfma_tm<T, 2>(p);
+    case 4: return mix_mfma_tm<T, 4>(p);
+    case 8: return mix_mfma_tm<T, 8>(p);
+    case 12: return mix_mfma_tm<T, 12>(p);
+    case 16: return mix_mfma_tm<T, 16>(p);
+  }
+  if constexpr (sizeof(T) == 8) return mix_group<T>(p.k, p.m) == 6 ? mix_mfma_tm<T, 6>(p) : mix_mfma_tm<T, 10>(p);
 }
 
 template <typename T>
@@ -1017,12 +1067,17 @@ bool mix_gram(int mode, T alpha, const Mvec<T>* V, const SdMat<T>* C, T beta, Mv
   p.gv = G ? G->dev() : nullptr;
   p.ldgv = G ? G->lda : 0;
   p.ngv = G ? G->nvec : 0;
-  const int ks = (k + 3) / 4;
-  int nparts;
-  if (ks <= 2) nparts = mix_gram_tm<T, 2>(p, !G);
-  else if (ks <= 4) nparts = mix_gram_tm<T, 4>(p, !G);
-  else if (ks <= 8) nparts = mix_gram_tm<T, 8>(p, !G);
-  else nparts = mix_gram_tm<T, 16>(p, !G);
+  int nparts = 0;
+  switch (mix_group<T>(k, m)) {
+    case 2: nparts = mix_gram_tm<T, 2>(p, !G); break;
+    case 4: nparts = mix_gram_tm<T, 4>(p, !G); break;
+    case 8: nparts = mix_gram_tm<T, 8>(p, !G); break;
+    case 12: nparts = mix_gram_tm<T, 12>(p, !G); break;
+    case 16: nparts = mix_gram_tm<T, 16>(p, !G); break;
+    default:
+      if constexpr (sizeof(T) == 8)
+        nparts = mix_group<T>(k, m) == 6 ? mix_gram_tm<T, 6>(p, !G) : mix_gram_tm<T, 10>(p, !G);
+  }
   const int na = G ? G->nvec : m, nout = na * m;
   hipLaunchKernelGGL(k_gram_finalize<T>, dim3(finalize_blocks(nout)), dim3(kBlock), 0, rt().stream, p.partials, nparts, na,
                      m, false, ga, gb, D->dev(), D->root->ld);

@@ -556,3 +556,52 @@ def test_fast_sync_same_results(be64, be32, dtype):
         assert np.array_equal(a, b)
     A.delete()
     m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("wide", [17, 24, 25, 33, 40, 41, 48, 49, 64, 65, 130])
+def test_wide_against_narrow(be64, be32, wide, dtype):
+    """Gram matrices of a wide block against 1..17 columns, either way round,
+    with beta, and W = alpha V C + beta W from the wide block, around the
+    column tiles (16, 32, 48, 64) and the lane groups' sizes, on blocks and on
+    column views that start unaligned, against FP64 sums"""
+    be = be64 if dtype == np.float64 else be32
+    eps = np.finfo(dtype).eps
+    n = 1003
+    rng = np.random.default_rng(wide)
+    V = rng.uniform(-1, 1, (n, wide + 1)).astype(dtype)
+    m = be.map(n)
+    vb = be.mvec(m, wide + 1, V)
+    for k in (1, 4, 15, 16, 17):
+        W = rng.uniform(-1, 1, (n, k + 1)).astype(dtype)
+        wb = be.mvec(m, k + 1, W)
+        for ofs in (0, 1):
+            v, w = vb.view(ofs, ofs + wide - 1), wb.view(ofs, ofs + k - 1)
+            Vd, Wd = V[:, ofs:ofs + wide].astype(float), W[:, ofs:ofs + k].astype(float)
+            for a, b, Ad, Bd in ((v, w, Vd, Wd), (w, v, Wd, Vd)):
+                C0 = rng.uniform(-1, 1, (Ad.shape[1], Bd.shape[1])).astype(dtype)
+                C = be.sdmat(*C0.shape, data=C0)
+                be.gram(1.5, a, b, -0.5, C)
+                want = 1.5 * Ad.T @ Bd - 0.5 * C0
+                bound = (n + 8) * eps * (1.5 * np.abs(Ad).T @ np.abs(Bd) + 0.5 * np.abs(C0))
+                assert np.all(np.abs(C.get() - want) <= bound), (k, ofs)
+                C.delete()
+            S0 = rng.uniform(-1, 1, (wide, k)).astype(dtype)
+            S = be.sdmat(wide, k, data=S0)
+            for beta in (0.0, 0.75):
+                out = be.mvec(m, k + 1, W)
+                o = out.view(ofs, ofs + k - 1)
+                be.times_sdmat(-1.25, v, S, beta, o)
+                got = out.get()
+                want = -1.25 * Vd @ S0.astype(float) + beta * Wd
+                bound = (wide + 8) * eps * (1.25 * np.abs(Vd) @ np.abs(S0.astype(float)) + beta * np.abs(Wd))
+                assert np.all(np.abs(got[:, ofs:ofs + k] - want) <= bound), (k, ofs, beta)
+                assert np.array_equal(got[:, k if ofs == 0 else 0], W[:, k if ofs == 0 else 0])
+                o.delete()
+                out.delete()
+            S.delete()
+            v.delete()
+            w.delete()
+        wb.delete()
+    vb.delete()
+    m.delete()
