@@ -15,6 +15,15 @@
 //                                                        system meeting only
 //                                                        its own columns
 //   h(i+1) = ||w||, v_{i+1} = w / h(i+1)
+// With the rotations on the device and a matrix of this library a step reads
+// the basis twice: the second update is late.  The product takes u_{i+1} =
+// w / h(i+1) from the w after the first update, and v_{i+1} = u_{i+1} - V e is
+// written in the next step's first sweep, which reads the basis anyway; its
+// norm follows from ||w||^2 - ||V'w||^2, and since A V = V H the product's
+// missing correction only changes the coefficients, h(0:i) -= H e.  The
+// sweeps are bound by the basis they read (2.1 M rows, 16 systems, FP64, 30
+// steps: 98.4 ms in three sweeps and a normalisation per step, 72.1 ms in two;
+// 5.1 TB/s in the sweeps).
 // (for more than 64 systems or m > 32: a Gram and a row mix of the whole
 // basis per pass, of which only the blocks' diagonals are used).
 //   Givens rotations of every system's Hessenberg column on the device (one
@@ -165,7 +174,7 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
     // the systems still iterating and the solution coefficients
     const bool cgs = rt().gmres_cgs && kk <= kGmresCgsMaxKk && m <= kGmresCgsMaxNl;
     const int64_t nrows = w->nrows, mk = (int64_t)m * kk;
-    const int64_t work_elems = cgs ? (int64_t)gmres_cgs_grid(nrows, kk) * mk + mk : 0;
+    const int64_t work_elems = cgs ? (int64_t)(gmres_cgs_grid(nrows, kk) + 1) * (mk + kk) : 0;
     const size_t dev_elems = cgs ? (size_t)(work_elems + 2 * mk + kk + kk + mk) : 0;
     TI* dbuf = cgs ? static_cast<TI*>(dev_alloc(sizeof(TI) * dev_elems)) : nullptr;
     struct Release {
@@ -196,7 +205,12 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
       const size_t m1 = (size_t)m + 1, nhd = (size_t)kk * m1 + 3 * (size_t)kk;
       const size_t nd = nhd + (size_t)kk * m * m1 + 2 * (size_t)kk * m;
       const size_t sbytes = nd * sizeof(double) + 3 * (size_t)kk * sizeof(int);
-      const size_t inv_off = (sbytes + 15) / 16 * 16, abytes = inv_off + sizeof(TI) * (size_t)kk;
+      // behind what comes back to the host: 1/norms (both forms), the unrotated
+      // Hessenberg matrices and two steps' corrections of the two-sweep cycle
+      const size_t inv_off = (sbytes + 15) / 16 * 16, dinv_off = inv_off + (sizeof(TI) * (size_t)kk + 15) / 16 * 16;
+      const size_t raw_off = dinv_off + sizeof(double) * (size_t)kk;
+      const size_t e_off = raw_off + sizeof(double) * (size_t)kk * m * m1;
+      const size_t abytes = e_off + 2 * sizeof(TI) * (size_t)mk;
       char* sbuf = static_cast<char*>(dev_alloc(abytes));
       struct ReleaseState {
         void* p;
@@ -217,6 +231,10 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
       ds.status = ip + kk;
       ds.iters0 = ip + 2 * kk;
       TI* d_inv = reinterpret_cast<TI*>(sbuf + inv_off);
+      double* d_dinv = reinterpret_cast<double*>(sbuf + dinv_off);
+      double* d_raw = reinterpret_cast<double*>(sbuf + raw_off);
+      TI* d_e[2] = {reinterpret_cast<TI*>(sbuf + e_off), reinterpret_cast<TI*>(sbuf + e_off) + mk};
+      Mvec<TI>* blk[2] = {vcur.get(), w.get()};  // two-sweep cycle: the product's input and result, in turn
       std::vector<double> hd(nhd, 0.0);
       std::vector<int> hi(3 * (size_t)kk, 0);
       for (int a = 0; a < kk; a++) {
@@ -237,20 +255,43 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
       upload_bytes(ds.steps, hi.data(), sizeof(int) * hi.size());
       uint32_t seqs[2] = {0, 0};
       for (; i < m; i++) {
-        op.apply_shifted(TI(1), s.data(), vcur.get(), TI(0), w.get(), nullptr);
-        project(w.get());
         const int nl = i + 1, nc = nl * kk;
         TI* D1 = d_outs;
         TI* D2 = d_outs + nc;
         TI* N = d_outs + 2 * nc;
-        const TI* v = Vb->dev();
+        TI* v = Vb->dev();
         const int64_t ldv = Vb->lda;
-        gmres_cgs_dev<TI>(0, nrows, v, ldv, w->dev(), w->lda, kk, nl, nullptr, nullptr, dbuf, work_elems, D1);
-        gmres_cgs_dev<TI>(1, nrows, v, ldv, w->dev(), w->lda, kk, nl, D1, d_act, dbuf, work_elems, D2);
-        gmres_cgs_dev<TI>(2, nrows, v, ldv, w->dev(), w->lda, kk, nl, D2, d_act, dbuf, work_elems, N);
-        gmres_givens_dev<TI>(ds, kk, m, i, d_outs, d_act, d_inv, 1000 * eps, maxIter);
-        View<TI> vn(Vb.get(), (i + 1) * kk, (i + 2) * kk - 1);
-        gmres_normalize_dev<TI>(nrows, kk, w->dev(), w->lda, d_inv, N, vcur->dev(), vcur->lda, vn->dev(), vn->lda);
+        if (op.A) {
+          // two sweeps: the product takes the vector before its second orthogonalisation, u_i = p_i / h
+          // (a factor per column), whose correction v_i = u_i - V e runs with the first dots, and its
+          // norm and e come from the sums of the step before; the rotations take the correction into the
+          // Hessenberg column, so that V and H satisfy the same Arnoldi relation
+          Mvec<TI>* x = blk[i % 2];
+          Mvec<TI>* y = blk[(i + 1) % 2];
+          SpmvRequest req;
+          req.has_shift = true;
+          if (i > 0) req.xscale = d_dinv;
+          req.xscale_stride = 1;
+          spmv_launch<TI>(op.A, TI(1), s.data(), x, TI(0), y, req, nullptr, nullptr);
+          project(y);
+          if (i == 0)
+            gmres_cgs_dev<TI>(0, nrows, v, ldv, y->dev(), y->lda, kk, 1, nullptr, nullptr, dbuf, work_elems, D1);
+          else
+            gmres_fix_dots_dev<TI>(nrows, v, ldv, x->dev(), x->lda, y->dev(), y->lda, kk, i, d_e[i % 2], d_dinv, dbuf,
+                                   work_elems, D1);
+          gmres_cgs_dev<TI>(4, nrows, v, ldv, y->dev(), y->lda, kk, nl, D1, d_act, dbuf, work_elems, D2);
+          gmres_givens_lag_dev<TI>(ds, d_raw, kk, m, i, d_outs, d_e[i % 2], d_e[(i + 1) % 2], d_act, d_dinv,
+                                   1000 * eps, maxIter);
+        } else {
+          op.apply_shifted(TI(1), s.data(), vcur.get(), TI(0), w.get(), nullptr);
+          project(w.get());
+          gmres_cgs_dev<TI>(0, nrows, v, ldv, w->dev(), w->lda, kk, nl, nullptr, nullptr, dbuf, work_elems, D1);
+          gmres_cgs_dev<TI>(1, nrows, v, ldv, w->dev(), w->lda, kk, nl, D1, d_act, dbuf, work_elems, D2);
+          gmres_cgs_dev<TI>(2, nrows, v, ldv, w->dev(), w->lda, kk, nl, D2, d_act, dbuf, work_elems, N);
+          gmres_givens_dev<TI>(ds, kk, m, i, d_outs, d_act, d_inv, 1000 * eps, maxIter);
+          View<TI> vn(Vb.get(), (i + 1) * kk, (i + 2) * kk - 1);
+          gmres_normalize_dev<TI>(nrows, kk, w->dev(), w->lda, d_inv, N, vcur->dev(), vcur->lda, vn->dev(), vn->lda);
+        }
         seqs[i % 2] = publish_async(d_act, sizeof(TI) * kk, 1 + i % 2);
         PHX_REQUIRE(seqs[i % 2] != 0, PHIST_FUNCTIONAL_ERROR, "GMRES: the active flags could not be published");
         if (i >= 1) {

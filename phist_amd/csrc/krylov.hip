@@ -506,6 +506,7 @@ void krylov_minres_step_dev(int64_t nrows, int k, int64_t ld, const T* v, T* vol
 //   mode 1: w(:,a) -= sum_l V(:,l*kk+a) C(l,a), then D(l,a) of the new w
 //   mode 2: as mode 1, then N(a) = ||new w(:,a)||^2
 //   mode 3: as mode 1 without outputs (x += V y at the end of a cycle)
+//   mode 4: as mode 1, then also N(a) = ||new w(:,a)||^2, after the D
 // with C(l,a) = coef[l*kk+a] where act[a] != 0, else 0 (act == nullptr: all).
 // Thread (rl, a) of a workgroup owns system a of row t*RP + rl (RP = 256/KP,
 // KP the next power of two >= kk) and keeps the row's nl basis entries in
@@ -534,7 +535,8 @@ __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
   const bool live = a < p.kk;
   // coefficients in LDS after the reduction area (registers hold the row's basis entries and the sums)
   // (zero for l >= nl, so the loads of those slots, which repeat vector nl-1, add nothing)
-  T* cf = sh + (MODE == 3 ? 0 : (MODE == 2 ? p.kk : p.nl * p.kk));
+  const int nout = MODE == 3 ? 0 : MODE == 2 ? p.kk : (p.nl + (MODE == 4)) * p.kk;
+  T* cf = sh + nout;
   if (MODE > 0) {
     for (int e = threadIdx.x; e < LMAX * p.kk; e += kBlock) {
       const int c = e % p.kk;
@@ -570,21 +572,25 @@ __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
     // keep every load of the row in flight together (the scheduler would otherwise pair each load with
     // its use to save registers, one memory latency per vector)
     __builtin_amdgcn_sched_barrier(0);
-    if (MODE > 0) {
+    if (MODE == 4) {  // four partial sums: one chain over the vectors is longer than the loads of a tile
+      T t[4] = {s, T(0), T(0), T(0)};
+#pragma unroll
+      for (int l = 0; l < LMAX; l++) t[l % 4] -= vv[l] * cf[l * p.kk + a];
+      s = (t[0] + t[1]) + (t[2] + t[3]);
+      *wr = s;
+    } else if (MODE > 0) {
 #pragma unroll
       for (int l = 0; l < LMAX; l++) s -= vv[l] * cf[l * p.kk + a];
       *wr = s;
     }
-    if (MODE == 0 || MODE == 1) {
+    if (MODE == 0 || MODE == 1 || MODE == 4) {
 #pragma unroll
       for (int l = 0; l < LMAX; l++) acc[l] += vv[l] * s;
-    } else if (MODE == 2) {
-      nacc += s * s;
     }
+    if (MODE == 2 || MODE == 4) nacc += s * s;
   }
   if (MODE == 3) return;
   // workgroup sums: lanes of a wave with the same a, then the waves in order
-  const int nout = MODE == 2 ? p.kk : p.nl * p.kk;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int nouts = MODE == 2 ? 1 : LMAX;
   if (MODE == 2) acc[0] = nacc;
@@ -592,6 +598,7 @@ __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
   for (int off = kp; off < 64; off <<= 1) {
 #pragma unroll
     for (int l = 0; l < nouts; l++) acc[l] += __shfl_xor(acc[l], off, 64);
+    if (MODE == 4) nacc += __shfl_xor(nacc, off, 64);
   }
 #pragma unroll 1
   for (int w = 0; w < kBlock / 64; w++) {
@@ -602,6 +609,10 @@ __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
           const int o = MODE == 2 ? a : l * p.kk + a;
           sh[o] = w == 0 ? acc[l] : sh[o] + acc[l];
         }
+      }
+      if (MODE == 4) {
+        const int o = p.nl * p.kk + a;
+        sh[o] = w == 0 ? nacc : sh[o] + nacc;
       }
     }
     __syncthreads();
@@ -629,6 +640,88 @@ static void cgs_lmax(CgsArgs<T> p, int grid, size_t lds) {
   }
 }
 
+// The pending basis vector and the first dots of a step, in one read of the
+// basis: v = p * inv - sum_l V(:, l) e(l) per system (0 where inv is 0, a
+// stopped system), written to basis slot nl, and with it D(l) = <V(:, l), w>
+// for the nl vectors before it and D(nl) = <v, w>.  Threads, loads and sums
+// as in k_gmres_cgs.
+template <typename T>
+struct FixArgs {
+  int64_t nrows, ntiles;
+  T* v;
+  int64_t ldv;
+  const T* p;
+  int64_t ldp;
+  const T* w;
+  int64_t ldw;
+  int kk, kp, nl;
+  const T* e;
+  const double* inv;
+  T* partials;
+};
+
+template <typename T, int LMAX>
+__global__ void __launch_bounds__(kBlock) k_gmres_fix_dots(const FixArgs<T> g) {
+  extern __shared__ unsigned char cgs_lds[];
+  T* sh = reinterpret_cast<T*>(cgs_lds);
+  const int kp = g.kp, rp = kBlock / kp;
+  const int a = threadIdx.x % kp, rl = threadIdx.x / kp;
+  const bool live = a < g.kk;
+  const int nout = (g.nl + 1) * g.kk;
+  T* cf = sh + nout;  // zero for l >= nl: those slots repeat vector nl-1
+  for (int q = threadIdx.x; q < LMAX * g.kk; q += kBlock) cf[q] = q < g.nl * g.kk ? g.e[q] : T(0);
+  __syncthreads();
+  const T inv = live ? (T)g.inv[a] : T(0);
+  T acc[LMAX], accv = T(0);
+#pragma unroll
+  for (int l = 0; l < LMAX; l++) acc[l] = T(0);
+  const TileWalk tw = xcd_tiles(g.ntiles);
+  for (int64_t t = tw.t; t < tw.end; t += tw.stride) {
+    const int64_t r = t * rp + rl;
+    if (!live || r >= g.nrows) continue;
+    const int64_t rows = g.nrows - t * rp < rp ? g.nrows - t * rp : rp;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        g.v + t * rp * g.ldv, (short)0, (int)(rows * g.ldv * (int64_t)sizeof(T)), 0x00020000);
+    const int vo = (int)((rl * g.ldv + a) * sizeof(T));
+    T vv[LMAX];
+#pragma unroll
+    for (int l = 0; l < LMAX; l++) {
+      const int so = (l < g.nl ? l : g.nl - 1) * g.kk * (int)sizeof(T);
+      if constexpr (sizeof(T) == 8)
+        vv[l] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0));
+      else
+        vv[l] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0));
+    }
+    const T pv = g.p[r * g.ldp + a], w = g.w[r * g.ldw + a];
+    __builtin_amdgcn_sched_barrier(0);  // every load of the row in flight together (k_gmres_cgs)
+    T s[4] = {inv * pv, T(0), T(0), T(0)};
+#pragma unroll
+    for (int l = 0; l < LMAX; l++) s[l % 4] -= vv[l] * cf[l * g.kk + a];
+    const T v = inv != T(0) ? (s[0] + s[1]) + (s[2] + s[3]) : T(0);
+    g.v[r * g.ldv + g.nl * g.kk + a] = v;
+#pragma unroll
+    for (int l = 0; l < LMAX; l++) acc[l] += vv[l] * w;
+    accv += v * w;
+  }
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int off = kp; off < 64; off <<= 1) {
+#pragma unroll
+    for (int l = 0; l < LMAX; l++) acc[l] += __shfl_xor(acc[l], off, 64);
+    accv += __shfl_xor(accv, off, 64);
+  }
+#pragma unroll 1
+  for (int w = 0; w < kBlock / 64; w++) {
+    if (wv == w && lane < kp && live) {
+#pragma unroll
+      for (int l = 0; l < LMAX; l++)
+        if (l < g.nl) sh[l * g.kk + a] = w == 0 ? acc[l] : sh[l * g.kk + a] + acc[l];
+      sh[g.nl * g.kk + a] = w == 0 ? accv : sh[g.nl * g.kk + a] + accv;
+    }
+    __syncthreads();
+  }
+  for (int o = threadIdx.x; o < nout; o += kBlock) g.partials[(int64_t)blockIdx.x * nout + o] = sh[o];
+}
+
 // Workgroups of a gmres_cgs_dev sweep (the partial sums need grid * nout
 // elements of work).
 int gmres_cgs_grid(int64_t nrows, int kk) {
@@ -641,7 +734,7 @@ int gmres_cgs_grid(int64_t nrows, int kk) {
 template <typename T>
 void gmres_cgs_dev(int mode, int64_t nrows, const T* v, int64_t ldv, T* w, int64_t ldw, int kk, int nl,
                    const T* coef, const T* act, T* work, int64_t work_elems, T* out) {
-  PHX_REQUIRE(kk >= 1 && kk <= kGmresCgsMaxKk && nl >= 1 && nl <= kGmresCgsMaxNl && mode >= 0 && mode <= 3,
+  PHX_REQUIRE(kk >= 1 && kk <= kGmresCgsMaxKk && nl >= 1 && nl <= kGmresCgsMaxNl && mode >= 0 && mode <= 4,
               PHIST_INVALID_INPUT, "Gram-Schmidt sweep over %d systems x %d vectors (mode %d)", kk, nl, mode);
   PHX_REQUIRE((int64_t)kBlock * ldv * (int64_t)sizeof(T) < (int64_t(1) << 31), PHIST_INVALID_INPUT,
               "basis row stride %ld too large", (long)ldv);  // a tile's rows fit one buffer resource
@@ -659,7 +752,7 @@ void gmres_cgs_dev(int mode, int64_t nrows, const T* v, int64_t ldv, T* w, int64
   p.act = act;
   p.partials = work;
   p.ntiles = (nrows + kBlock / p.kp - 1) / (kBlock / p.kp);
-  const int nout = mode == 2 ? kk : nl * kk;
+  const int nout = mode == 2 ? kk : (nl + (mode == 4)) * kk;
   const int grid = gmres_cgs_grid(nrows, kk);
   PHX_REQUIRE(mode == 3 || (int64_t)grid * nout + nout <= work_elems, PHIST_FUNCTIONAL_ERROR,
               "Gram-Schmidt work of %ld elements is too small", (long)work_elems);
@@ -669,7 +762,43 @@ void gmres_cgs_dev(int mode, int64_t nrows, const T* v, int64_t ldv, T* w, int64
     case 0: cgs_lmax<T, 0>(p, grid, lds); break;
     case 1: cgs_lmax<T, 1>(p, grid, lds); break;
     case 2: cgs_lmax<T, 2>(p, grid, lds); break;
+    case 4: cgs_lmax<T, 4>(p, grid, lds); break;
     default: cgs_lmax<T, 3>(p, grid, lds); return;
+  }
+  hipLaunchKernelGGL(k_reduce_partials<T>, dim3((nout + 15) / 16), dim3(kBlock), 0, rt().stream, work, grid, nout,
+                     out);
+  PHX_HIP(hipGetLastError());
+}
+
+template <typename T, int LMAX>
+static void fix_launch(const FixArgs<T>& g, int grid) {
+  const size_t lds = sizeof(T) * ((size_t)(g.nl + 1) * g.kk + (size_t)LMAX * g.kk);
+  hipLaunchKernelGGL((k_gmres_fix_dots<T, LMAX>), dim3(grid), dim3(kBlock), lds, rt().stream, g);
+  PHX_HIP(hipGetLastError());
+}
+
+template <typename T>
+void gmres_fix_dots_dev(int64_t nrows, T* v, int64_t ldv, const T* p, int64_t ldp, const T* w, int64_t ldw, int kk,
+                        int nl, const T* e, const double* inv, T* work, int64_t work_elems, T* out) {
+  PHX_REQUIRE(kk >= 1 && kk <= kGmresCgsMaxKk && nl >= 1 && nl < kGmresCgsMaxNl, PHIST_INVALID_INPUT,
+              "basis step over %d systems x %d vectors", kk, nl);
+  PHX_REQUIRE((int64_t)kBlock * ldv * (int64_t)sizeof(T) < (int64_t(1) << 31), PHIST_INVALID_INPUT,
+              "basis row stride %ld too large", (long)ldv);
+  FixArgs<T> g{nrows, 0, v, ldv, p, ldp, w, ldw, kk, 1, nl, e, inv, work};
+  while (g.kp < kk) g.kp <<= 1;
+  g.ntiles = (nrows + kBlock / g.kp - 1) / (kBlock / g.kp);
+  const int nout = (nl + 1) * kk, grid = gmres_cgs_grid(nrows, kk);
+  PHX_REQUIRE((int64_t)grid * nout + nout <= work_elems, PHIST_FUNCTIONAL_ERROR,
+              "basis step work of %ld elements is too small", (long)work_elems);
+  switch ((nl + 3) / 4) {
+    case 1: fix_launch<T, 4>(g, grid); break;
+    case 2: fix_launch<T, 8>(g, grid); break;
+    case 3: fix_launch<T, 12>(g, grid); break;
+    case 4: fix_launch<T, 16>(g, grid); break;
+    case 5: fix_launch<T, 20>(g, grid); break;
+    case 6: fix_launch<T, 24>(g, grid); break;
+    case 7: fix_launch<T, 28>(g, grid); break;
+    default: fix_launch<T, 32>(g, grid); break;
   }
   hipLaunchKernelGGL(k_reduce_partials<T>, dim3((nout + 15) / 16), dim3(kBlock), 0, rt().stream, work, grid, nout,
                      out);
@@ -733,6 +862,98 @@ __global__ void __launch_bounds__(64) k_gmres_givens(GmresDevState st, int kk, i
     act[a] = T(0);
     st.status[a] = 3;
   }
+}
+
+// Step i of the two-sweep cycle (gmres.cpp), one wave per system a, lane r
+// for row r of the Hessenberg column: from outs = D1 | D2 | N ((i+1)*kk first
+// dots, (i+1)*kk dots after the update, the squared norms of the updated w)
+// and the step before's correction e_in (v_i = u_i - V e_in, u_i the vector
+// the product was formed with)
+//   h(i+1,i)^2 = N - ||D2||^2      (w - V D2, V orthonormal; at least eps N,
+//                                   the rounding of that difference)
+//   h(0:i,i)   = D1 + D2 - H(0:i, 0:i-1) e_in
+// then the rotations and the stopping test of k_gmres_givens.  Writes inv[a] =
+// 1 / h(i+1,i), rounded to T (0 for a stopped system), and e_out = D2 inv.
+template <typename T>
+__global__ void __launch_bounds__(64) k_gmres_givens_lag(GmresDevState st, double* __restrict__ Hraw, int kk, int m,
+                                                         int i, const T* __restrict__ outs,
+                                                         const T* __restrict__ e_in, T* __restrict__ e_out, T* act,
+                                                         double* __restrict__ inv, double eps1000, int max_iter) {
+  __shared__ double h[kGmresCgsMaxNl + 1], cs[kGmresCgsMaxNl], sn[kGmresCgsMaxNl];
+  const int a = blockIdx.x, r = threadIdx.x, nc = (i + 1) * kk, m1 = m + 1;
+  const bool live = act[a] != T(0);
+  const double d2 = r <= i ? (double)outs[nc + r * kk + a] : 0.0;
+  const double nrm2 = (double)outs[2 * nc + a];
+  const double eps = sizeof(T) == 8 ? 2.220446049250313e-16 : 1.1920928955078125e-07;
+  const double hn = sqrt(fmax(nrm2 - wave_sum_strided<1>(d2 * d2), eps * nrm2));
+  const bool ok = isfinite(nrm2) && isfinite(hn);
+  const T f = live && ok && hn > 0.0 ? T(1.0 / hn) : T(0);
+  if (r <= i) e_out[r * kk + a] = f != T(0) ? T(d2 * (double)f) : T(0);
+  if (r == 0) inv[a] = (double)f;
+  if (!live) return;  // the whole wave (live is uniform)
+  if (!ok) {
+    if (r == 0) {
+      act[a] = T(0);
+      st.status[a] = 3;
+    }
+    return;
+  }
+  if (r <= m) {
+    double x = 0.0;
+    if (r <= i) {
+      x = (double)outs[r * kk + a] + d2;
+      for (int c = 0; c < i; c++) x -= Hraw[((size_t)a * m + c) * m1 + r] * (double)e_in[c * kk + a];
+    } else if (r == i + 1) {
+      x = hn;
+    }
+    h[r] = x;
+    Hraw[((size_t)a * m + i) * m1 + r] = x;
+    if (r < i) {
+      cs[r] = st.cs[(size_t)a * m + r];
+      sn[r] = st.sn[(size_t)a * m + r];
+    }
+  }
+  __syncthreads();
+  if (r == 0) {
+    for (int l = 0; l < i; l++) {
+      const double p0 = h[l], p1 = h[l + 1];
+      h[l] = cs[l] * p0 + sn[l] * p1;
+      h[l + 1] = -sn[l] * p0 + cs[l] * p1;
+    }
+    const double p0 = h[i], p1 = h[i + 1];
+    const double q = hypot(p0, p1);
+    const double c = q > 0.0 ? p0 / q : 1.0, s = q > 0.0 ? p1 / q : 0.0;
+    st.cs[(size_t)a * m + i] = c;
+    st.sn[(size_t)a * m + i] = s;
+    h[i] = q;
+    h[i + 1] = 0.0;
+    double* g = st.g + (size_t)a * m1;
+    const double gi = g[i];
+    g[i + 1] = -s * gi;
+    g[i] = c * gi;
+    st.steps[a] = i + 1;
+    const double nr = fabs(s * gi);
+    const double rel = nr / st.normR0[a];
+    st.relres[a] = rel;
+    if (nr < eps1000 || rel < st.tol[a] || hn == 0.0) {
+      act[a] = T(0);
+      st.status[a] = 0;
+    } else if (st.iters0[a] + i + 1 >= max_iter) {
+      act[a] = T(0);
+      st.status[a] = 3;
+    }
+  }
+  __syncthreads();
+  if (r <= m) st.H[((size_t)a * m + i) * m1 + r] = h[r];
+}
+
+template <typename T>
+void gmres_givens_lag_dev(const GmresDevState& st, double* Hraw, int kk, int m, int i, const T* outs, const T* e_in,
+                          T* e_out, T* act, double* inv, double eps1000, int max_iter) {
+  PHX_REQUIRE(kk >= 1 && kk <= 64 && m <= kGmresCgsMaxNl, PHIST_INVALID_INPUT, "%d systems, basis of %d", kk, m);
+  hipLaunchKernelGGL(k_gmres_givens_lag<T>, dim3(kk), dim3(64), 0, rt().stream, st, Hraw, kk, m, i, outs, e_in, e_out,
+                     act, inv, eps1000, max_iter);
+  PHX_HIP(hipGetLastError());
 }
 
 // v = w * inv (column a by inv[a]; 0 where ||w(:,a)||^2 = nrm2[a] is not
@@ -843,6 +1064,14 @@ template void gmres_cgs_dev<double>(int, int64_t, const double*, int64_t, double
                                     const double*, const double*, double*, int64_t, double*);
 template void gmres_cgs_dev<float>(int, int64_t, const float*, int64_t, float*, int64_t, int, int, const float*,
                                    const float*, float*, int64_t, float*);
+template void gmres_fix_dots_dev<double>(int64_t, double*, int64_t, const double*, int64_t, const double*, int64_t, int,
+                                         int, const double*, const double*, double*, int64_t, double*);
+template void gmres_fix_dots_dev<float>(int64_t, float*, int64_t, const float*, int64_t, const float*, int64_t, int,
+                                        int, const float*, const double*, float*, int64_t, float*);
+template void gmres_givens_lag_dev<double>(const GmresDevState&, double*, int, int, int, const double*, const double*,
+                                           double*, double*, double*, double, int);
+template void gmres_givens_lag_dev<float>(const GmresDevState&, double*, int, int, int, const float*, const float*,
+                                          float*, float*, double*, double, int);
 template void gmres_givens_dev<double>(const GmresDevState&, int, int, int, const double*, double*, double*, double,
                                        int);
 template void gmres_givens_dev<float>(const GmresDevState&, int, int, int, const float*, float*, float*, double, int);

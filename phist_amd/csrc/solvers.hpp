@@ -25,14 +25,25 @@ void convert_block(const TS* x, int64_t ldx, TD* y, int64_t ldy, int64_t nrows, 
 // by side (column l*kk + a of v: vector l of system a), one read of the basis
 // each; mode 0: out(l,a) = <v(:,l*kk+a), w(:,a)>; 1: w(:,a) -= sum_l
 // v(:,l*kk+a) c(l,a), then out as in mode 0 for the new w; 2: the update,
-// then out(a) = ||w(:,a)||^2; 3: the update only.  c(l,a) = coef[l*kk+a]
+// then out(a) = ||w(:,a)||^2; 3: the update only; 4: as 1, then also the
+// squared norms.  c(l,a) = coef[l*kk+a]
 // (device) where act[a] != 0 (act == nullptr: every system).  work holds
 // gmres_cgs_grid(nrows, kk) * nout partial sums plus nout; out (device) gets
-// the nout = nl*kk (mode 2: kk) sums.
+// the nout = nl*kk (mode 2: kk, mode 4: (nl+1)*kk) sums.
 int gmres_cgs_grid(int64_t nrows, int kk);
 template <typename T>
 void gmres_cgs_dev(int mode, int64_t nrows, const T* v, int64_t ldv, T* w, int64_t ldw, int kk, int nl,
                    const T* coef, const T* act, T* work, int64_t work_elems, T* out);
+
+// basis vector nl completed from its pending block (v = p inv - V e), and the
+// dots of w with it and the nl vectors before it; then a step's Givens
+// rotations from the lagged sums (krylov.hip)
+template <typename T>
+void gmres_fix_dots_dev(int64_t nrows, T* v, int64_t ldv, const T* p, int64_t ldp, const T* w, int64_t ldw, int kk,
+                        int nl, const T* e, const double* inv, T* work, int64_t work_elems, T* out);
+template <typename T>
+void gmres_givens_lag_dev(const GmresDevState& st, double* Hraw, int kk, int m, int i, const T* outs, const T* e_in,
+                          T* e_out, T* act, double* inv, double eps1000, int max_iter);
 
 // device Givens step and basis normalisation of the blocked GMRES (krylov.hip; GmresDevState in amd_common.hpp)
 template <typename T>

@@ -157,3 +157,45 @@ def test_gmres_device_givens_matches_host(be64, restart, nsys, tol):
         bound = np.where(it1 == it0, 1e-4 if fp32 else 1e-8, 20 * t)
         assert np.all(np.linalg.norm(x1 - x0, axis=0) <= bound * scale), (it0, it1)
     A.delete()
+
+
+@pytest.mark.parametrize("restart,nsys", [(1, 3), (2, 1), (4, 64), (5, 33), (32, 2), (31, 5)])
+def test_gmres_two_sweep_cycle(be64, restart, nsys):
+    """the two-sweep cycle (second orthogonalisation one step late) against
+    the host rotations' three sweeps around the sizes of its register slots
+    and system groups: iteration counts within one, the tolerance by the true
+    residual, for a band and for a diagonal of three values, whose Krylov
+    space ends after three steps"""
+    import ctypes
+
+    import phist_amd
+    fl = ctypes.c_int(0)
+
+    @phist_amd.ROWFUNC
+    def three(i, nnz, cols, vals, arg):
+        nnz[0], cols[0] = 1, i
+        ctypes.cast(vals, ctypes.POINTER(ctypes.c_double))[0] = 2.0 + i % 3
+        return 0
+
+    for A in (be64.banded_random(3001, 9, 80, 25.0, 5), be64.from_rowfunc(3001, 1, three, None)):
+        n = A.nrows
+        shifts = np.linspace(0.0, 4.0, nsys)
+        Bh = np.random.default_rng(restart).uniform(-1, 1, (n, nsys))
+        Bh[:, nsys // 2] *= nsys > 1  # one system without a right-hand side
+        its = {}
+        try:
+            for dev in (0, 1):
+                be64.L.phist_amd_set_gmres_device(dev, ctypes.byref(fl))
+                B, X = be64.mvec(A.domain_map, nsys, Bh), be64.mvec(A.domain_map, nsys)
+                it, rr, unconv = be64.gmres_shifted(A, shifts, B, X, 1e-9, 500, restart=restart)
+                assert unconv == 0
+                live = [j for j in range(nsys) if np.any(Bh[:, j])]
+                got = true_relres(A, shifts[live], Bh[:, live], X.get()[:, live])
+                assert np.all(got <= 2e-9), (dev, got)
+                its[dev] = it
+                B.delete()
+                X.delete()
+        finally:
+            be64.L.phist_amd_set_gmres_device(1, ctypes.byref(fl))
+        assert np.all(np.abs(its[0] - its[1]) <= 1), its
+        A.delete()
