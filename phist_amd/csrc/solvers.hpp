@@ -236,7 +236,8 @@ void copy_any(const Mvec<TS>* X, Mvec<TD>* Y) {
 // MINRES with Paige & Saunders' short recurrences.  Per iteration: one
 // shifted SpMV whose fused <v, Av> dots give the Lanczos alphas, the
 // projection, k_lanczos (update + norms) and k_minres (direction, solution,
-// next Lanczos vector).  A slot whose system has converged (|phibar| <=
+// next Lanczos vector; on the device path every other iteration runs the
+// updates of two, k_minres2).  A slot whose system has converged (|phibar| <=
 // tol*|b|), broken down or reached its iteration limit stops updating; its
 // solution can be stored and the slot loaded with the next system while the
 // others keep iterating (the slot swap of
@@ -254,8 +255,12 @@ void copy_any(const Mvec<TS>* X, Mvec<TD>* Y) {
 // ---------------------------------------------------------------------------
 template <typename T>
 void krylov_minres_step_dev(int64_t nrows, int k, int64_t ld, const T* v, T* vold, T* w, const T* d1, T* d2, T* x,
-                            const T* dots, MinresState* st, T* work, const T* Q = nullptr, int64_t ldq = 0,
-                            int nq = 0, const T* C = nullptr, int ldc = 0, int phase = -1, int nact = -1);
+                            const T* dots, MinresState* st, T* coef, const T* Q, int64_t ldq, int nq, const T* C,
+                            int ldc, int phase, int nact, bool update);
+// the direction and solution update of one iteration (coef1 null) or of two
+template <typename T>
+void krylov_minres_update_dev(int64_t nrows, int k, int64_t ld, const T* v0, const T* coef0, const double* scale0,
+                              const T* v1, const T* coef1, const double* scale1, T* d1, T* d2, T* x, int nact);
 
 // device column states of freshly loaded systems (see krylov.hip)
 template <typename T>
@@ -273,16 +278,13 @@ class MinresBatch {
     // six separate blocks of `cap` columns (row stride cap each): the SpMV
     // gathers rows of V, and a V whose rows are interleaved with the other
     // blocks would waste most of every cache line it touches
-    for (int b = 0; b < 6; b++) {
-      blk_[b].p = api::mvec_create<T>(map, cap);
-      blas_put_value<T>(blk_[b].p, T(0));
-    }
+    for (int b = 0; b < 6; b++) blk_[b].p = api::mvec_create<T>(map, cap);  // zero
     if (Q_ && Q_->nvec > 0) C_.reset(new SdBox<T>(Q_->nvec, cap));
     dev_ = op_.A != nullptr && rt().minres_device;
     if (dev_) {
       d_st_ = static_cast<MinresState*>(dev_alloc(sizeof(MinresState) * cap));
       d_dots_ = static_cast<T*>(dev_alloc(sizeof(T) * 2 * cap));
-      d_work_ = static_cast<T*>(dev_alloc(sizeof(T) * 8 * cap));
+      d_work_ = static_cast<T*>(dev_alloc(sizeof(T) * kWork * cap));
       d_shift_ = static_cast<T*>(dev_alloc(sizeof(T) * cap));
       h_buf_ = static_cast<MinresState*>(pinned_alloc(sizeof(MinresState) * 3 * cap));
       h_shift_ = static_cast<T*>(pinned_alloc(sizeof(T) * cap));
@@ -300,7 +302,7 @@ class MinresBatch {
       drop_graphs();
       if (garena_) dev_release(garena_, garena_bytes_);
       dev_release(d_shift_, sizeof(T) * cap_);
-      dev_release(d_work_, sizeof(T) * 8 * cap_);
+      dev_release(d_work_, sizeof(T) * kWork * cap_);
       dev_release(d_dots_, sizeof(T) * 2 * cap_);
       dev_release(d_st_, sizeof(MinresState) * cap_);
     } catch (...) {
@@ -345,10 +347,13 @@ class MinresBatch {
     const int k = B->nvec;
     PHX_REQUIRE(k == cap_, PHIST_INVALID_INPUT, "load_all needs %d columns", cap_);
     drain();
+    finish_update();
     if (dev_ && B->nrows > 0) {
       // no host round trip: b stays unnormalised in v (factor 1/||b|| in the
       // column state), the norms go from the device dots into the states
-      for (int r : {VOLD, D1, D2, XS}) blas_put_value<T>(cur(r), T(0));
+      if (!fresh_)
+        for (int r : {VOLD, D1, D2, XS}) blas_put_value<T>(cur(r), T(0));
+      fresh_ = false;
       copy_any<TS, T>(B, cur(V));
       blas_dot_dev<T>(cur(V), cur(V), d_work_);
       for (int j = 0; j < k; j++) start(j, 1.0, shifts[j], tol[j], max_iter[j]);  // the norms follow on the device
@@ -373,6 +378,8 @@ class MinresBatch {
   // slot j from column c of B (x = 0)
   template <typename TS>
   void load(int j, const Mvec<TS>* B, int c, T shift, double tol, int max_iter) {
+    finish_update();
+    fresh_ = false;
     if (dev_ && B->nrows > 0) {  // as load_all: no host round trip
       for (int r : {VOLD, D1, D2, XS}) {
         View<T> col(cur(r), j, j);
@@ -405,16 +412,19 @@ class MinresBatch {
 
   // solution of slot j into column c of X (any precision)
   template <typename TD>
-  void store(int j, Mvec<TD>* X, int c) const {
+  void store(int j, Mvec<TD>* X, int c) {
+    finish_update();
     View<T> xj(cur(XS), j, j);
     View<TD> xc(X, c, c);
     copy_any<T, TD>(xj.get(), xc.get());
   }
   template <typename TD>
-  void store_all(Mvec<TD>* X) const {
+  void store_all(Mvec<TD>* X) {
+    finish_update();
     copy_any<T, TD>(cur(XS), X);
   }
   void release(int j) {
+    finish_update();
     st_[j] = Slot();
     if (dev_) upload(j, 1);  // frozen on the device as well
   }
@@ -520,11 +530,34 @@ class MinresBatch {
       gemm_gram<T>(T(1), Q_, w, T(0), C_->get(), false);
       if (!fuse) gemm_times_sd<T>(T(-1), Q_, C_->get(), T(1), w);
     }
+    // The direction and solution updates wait for the next iteration's, which then does both in one pass
+    // (k_minres2: v is the next v_old, so no block is kept longer); a captured iteration does its own.
+    const bool now = rt().capturing;
     krylov_minres_step_dev<T>(v->nrows, k, cap_, v->dev(), cur(VOLD)->dev(), w->dev(), cur(D1)->dev(),
-                              cur(D2)->dev(), cur(XS)->dev(), d_dots_, d_st_, d_work_, fuse ? Q_->dev() : nullptr,
+                              cur(D2)->dev(), cur(XS)->dev(), d_dots_, d_st_, coef(ph), fuse ? Q_->dev() : nullptr,
                               fuse ? Q_->lda : 0, fuse ? Q_->nvec : 0, fuse ? C_->get()->dev() : nullptr,
-                              fuse ? C_->get()->root->ld : 0, ph, nact);
+                              fuse ? C_->get()->root->ld : 0, ph, nact, now);
+    if (!now && waiting_) {
+      // (the directions' roles have swapped once since the waiting iteration)
+      const int nboth = nact < 0 || wait_nact_ < 0 ? -1 : std::max(nact, wait_nact_);
+      const int po = (int)((phase_ + 2) % 3);
+      krylov_minres_update_dev<T>(v->nrows, k, cap_, cur(VOLD)->dev(), coef(po), &d_st_[0].sc[po], v->dev(), coef(ph),
+                                  &d_st_[0].sc[ph], cur(D2)->dev(), cur(D1)->dev(), cur(XS)->dev(), nboth);
+      waiting_ = false;
+    } else if (!now) {
+      waiting_ = true;
+      wait_nact_ = nact;
+    }
     advance_roles();
+  }
+  T* coef(int phase) const { return d_work_ + (size_t)(1 + 5 * phase) * cap_; }
+  // the update of an iteration that waits for a next one
+  void finish_update() {
+    if (!waiting_) return;
+    waiting_ = false;
+    const int po = (int)((phase_ + 2) % 3);  // that iteration's v is v_old by now
+    krylov_minres_update_dev<T>(cur(VOLD)->nrows, cap_, cap_, cur(VOLD)->dev(), coef(po), &d_st_[0].sc[po], nullptr,
+                                nullptr, nullptr, cur(D2)->dev(), cur(D1)->dev(), cur(XS)->dev(), wait_nact_);
   }
   // after a device iteration: w (unnormalised) is the next v, v the next
   // v_old, the old v_old block takes the next SpMV; the direction blocks swap
@@ -633,6 +666,7 @@ class MinresBatch {
         const int p = (int)(phase_ % 6);  // the layout of the rotating blocks and factors
         if (!gexec_[p]) capture(p);
         if (gexec_[p]) {
+          finish_update();
           PHX_HIP(hipGraphLaunch(gexec_[p], r.stream));
           r.graph_launches++;
           for (int t = 0; t < glen_; t++) advance_roles();
@@ -722,7 +756,11 @@ class MinresBatch {
   bool dev_ = false;
   MinresState* d_st_ = nullptr;
   T* d_dots_ = nullptr;
+  static constexpr int kWork = 16;  // per column: a norm, then the update coefficients of three phases
   T* d_work_ = nullptr;
+  bool fresh_ = true;     // every block is as created, zero
+  bool waiting_ = false;  // the last iteration's direction and solution update is not enqueued yet
+  int wait_nact_ = -1;    // ... and its columns
   T* d_shift_ = nullptr;
   MinresState* h_buf_ = nullptr;  // pinned: two lagged state copies, then the upload staging
   T* h_shift_ = nullptr;          // pinned staging of the shifts

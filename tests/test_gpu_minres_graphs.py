@@ -130,3 +130,34 @@ def test_serve_graphs_bitexact(be64, graphs):
         assert it0 == it1 and np.array_equal(X0, X1)
     A1.delete()
     A2.delete()
+
+
+@pytest.mark.parametrize("iters", [1, 2, 3, 8])
+@pytest.mark.parametrize("k", [1, 3, 8, 33])
+def test_paired_updates_equal_single_ones(be64, k, iters):
+    """the direction and solution updates of two iterations in one pass give
+    bit for bit those of one pass per iteration (captured iterations do their
+    own), for even and odd numbers of iterations, whole vectors and ragged
+    widths, FP64 and FP32, and with fewer slots than systems"""
+    A = be64.honeycomb(31, 29, 0, 0, 0, 1.0, 7)
+    n = A.nrows
+    shifts = np.linspace(-2.0, 2.5, k)
+    B = be64.mvec(A.domain_map, k, np.random.default_rng(k).uniform(-1, 1, (n, k)))
+    out = {}
+    try:
+        for graphs in (False, True):
+            be64.set_minres_graphs(graphs, 1, 1)
+            X, Y, Z = (be64.mvec(A.domain_map, k) for _ in range(3))
+            be64.minres_shifted(A, shifts, B, X, 1e-13, iters)
+            be64.minres_shifted(A, shifts, B, Y, 1e-13, iters, fp32=True)
+            be64.minres_refill(A, shifts, B, Z, 1e-13, iters, max(1, k // 2))
+            out[graphs] = [v.get() for v in (X, Y, Z)]
+            for v in (X, Y, Z):
+                v.delete()
+    finally:
+        be64.set_minres_graphs(False)
+    for a, b in zip(out[False], out[True]):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+    assert np.all(np.linalg.norm(out[False][0], axis=0) > 0)
+    B.delete()
+    A.delete()
