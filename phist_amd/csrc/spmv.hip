@@ -885,7 +885,8 @@ inline bool spmv_long_rows(const SparseMat<T>* A) {
 //    +-3000: 93 in one, 70 in two), from 128 bytes on b4 (601 / 629)
 //  - rows of at most 8 entries (a 3D stencil): one batch; x rows of 32 bytes
 //    in one lane (64 x 58 x 51 grid: 5.9 against 6.8, 128^3 shifted: 66 /
-//    79), from 64 bytes on b4 (128^3, 8 columns: 106 at b4, 111 at b6; 16:
+//    79) unless that leaves the chip without waves (below 128 Ki rows, two
+//    per SIMD; 32^3 with dots 6.9 against 5.8), from 64 bytes on b4 (128^3, 8 columns: 106 at b4, 111 at b6; 16:
 //    213 / 219), shifted only from 128 (8 columns 143 at b4, 125 at b6)
 //  - rows of at most 4 entries (a sheet): x rows of 128 bytes and more in
 //    32-byte lanes, b3 (8 M rows, 32 columns: 1092 against 1470 in 16-byte
@@ -911,7 +912,7 @@ SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
       d.lane_bytes = rb >= 128 ? 32 : 0;
     }
   } else if (A->max_row_len > 4) {
-    d.lane_bytes = rb == 32 || rb >= 256 ? 32 : 0;
+    d.lane_bytes = (rb == 32 && A->nrows >= (1 << 17)) || rb >= 256 ? 32 : 0;
     d.blocks_per_cu = rb >= (full ? 128 : 64) ? 4 : 6;
   } else {
     d.lane_bytes = rb >= 128 ? 32 : 0;
