@@ -11,9 +11,9 @@
 //
 // Same mapping as the SpMV: a row is owned by LPR lanes holding VPL
 // consecutive columns each, workgroups walk row tiles on a persistent
-// XCD-aware grid, reductions are fixed-order two-stage.  The streaming
-// kernels take kRowUnroll rows per lane group and tile, whose loads are all
-// in flight before the first store.
+// XCD-aware grid, reductions are fixed-order two-stage.  They
+// take kRowUnroll rows per lane group and tile, whose loads are all
+// in flight before the first store or product.
 #include "amd_device.hpp"
 #include <algorithm>
 
@@ -37,8 +37,11 @@ struct RowArgs {
 
 enum : int { B_READX = 1, B_READY = 2 };
 
-// rows per lane group and tile of the streaming kernels (k_axpby, k_elemwise)
+// rows per lane group and tile
 constexpr int kRowUnroll = 4;
+// workgroups per CU of the dots: with four rows under way per lane group four
+// keep HBM busy, and the partial sums are half as many as with eight
+constexpr int kDotBlocksPerCu = 4;
 
 template <typename T, int VPL, int LPR>
 __global__ void __launch_bounds__(kBlock) k_axpby(const RowArgs<T> p) {
@@ -121,15 +124,24 @@ __global__ void __launch_bounds__(kBlock) k_coldot(const RowArgs<T> p) {
   T acc[VPL];
 #pragma unroll
   for (int e = 0; e < VPL; e++) acc[e] = T(0);
+  const bool self = p.x == p.y && p.ldx == p.ldy;  // a norm reads its block once
   const TileWalk tw = xcd_tiles(p.ntiles);
   for (int64_t t = tw.t; t < tw.end; t += tw.stride) {
-    const int64_t i = t * RPB + wv * RPW + rw;
-    if (i >= p.nrows || !colok) continue;
-    T xv[VPL], yv[VPL];
-    vload<T, VPL>(p.x + i * p.ldx + c0, xv);
-    vload<T, VPL>(p.y + i * p.ldy + c0, yv);
+    T xv[kRowUnroll][VPL], yv[kRowUnroll][VPL];
 #pragma unroll
-    for (int e = 0; e < VPL; e++) acc[e] = fma(xv[e], yv[e], acc[e]);
+    for (int u = 0; u < kRowUnroll; u++) {
+      const int64_t i = (t * kRowUnroll + u) * RPB + wv * RPW + rw;
+#pragma unroll
+      for (int e = 0; e < VPL; e++) xv[u][e] = yv[u][e] = T(0);
+      if (i < p.nrows && colok) {
+        vload<T, VPL>(p.x + i * p.ldx + c0, xv[u]);
+        if (!self) vload<T, VPL>(p.y + i * p.ldy + c0, yv[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kRowUnroll; u++)
+#pragma unroll
+      for (int e = 0; e < VPL; e++) acc[e] = fma(xv[u][e], self ? xv[u][e] : yv[u][e], acc[e]);
   }
   __shared__ T red[kBlock / 64][64 * VPL];
 #pragma unroll
@@ -156,7 +168,7 @@ enum Kind { K_AXPBY, K_ELEM, K_DOT };
 template <typename T, int VPL, int LPR>
 int launch_kind(Kind kind, RowArgs<T>& p) {
   constexpr int RPB = (kBlock / 64) * (64 / LPR);
-  const int64_t rows_per_tile = kind == K_DOT ? RPB : (int64_t)RPB * kRowUnroll;
+  const int64_t rows_per_tile = (int64_t)RPB * kRowUnroll;
   p.ntiles = (p.nrows + rows_per_tile - 1) / rows_per_tile;
   int grid;
   ktimer_begin();
@@ -170,7 +182,7 @@ int launch_kind(Kind kind, RowArgs<T>& p) {
       hipLaunchKernelGGL((k_elemwise<T, VPL, LPR>), dim3(grid), dim3(kBlock), 0, rt().stream, p);
       break;
     default:
-      grid = persistent_blocks(k_coldot<T, VPL, LPR>, 0, p.ntiles);
+      grid = reducing_blocks(k_coldot<T, VPL, LPR>, 0, p.ntiles, kDotBlocksPerCu);
       p.partials = (T*)device_work(sizeof(T) * ((size_t)grid * p.ncols + p.ncols));
       hipLaunchKernelGGL((k_coldot<T, VPL, LPR>), dim3(grid), dim3(kBlock), 0, rt().stream, p);
       break;

@@ -360,7 +360,7 @@ int gram_launch_one(GramArgs<T>& g) {
   constexpr int RPB = (kBlock / 64) * (64 / LPR);
   g.ntiles = (g.nrows + RPB - 1) / RPB;
   const size_t lds = sizeof(T) * g.na * g.nb;
-  const int grid = persistent_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
+  const int grid = reducing_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
   g.partials = (T*)device_work(sizeof(T) * (size_t)grid * g.na * g.nb);
   ktimer_begin();
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, rt().stream, g);
@@ -375,7 +375,7 @@ int gram_rows_launch(GramArgs<T>& g) {
   constexpr int RPB = (kBlock / 64) * (64 / LPR);
   g.ntiles = (g.nrows + RPB - 1) / RPB;
   const size_t lds = sizeof(T) * g.na * g.nb;
-  const int grid = persistent_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
+  const int grid = reducing_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
   g.partials = (T*)device_work(sizeof(T) * (size_t)grid * g.na * g.nb);
   ktimer_begin();
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, rt().stream, g);
@@ -411,7 +411,7 @@ static int gram_mfma_launch(GramArgs<T>& g) {
   auto kern = k_gram_mfma<T, TM, TK, SELF, PAIR>;
   g.ntiles = (g.nrows + 63) / 64;
   const size_t lds = sizeof(T) * g.na * g.nb;
-  const int grid = persistent_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
+  const int grid = reducing_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
   g.partials = (T*)device_work(sizeof(T) * (size_t)grid * g.na * g.nb);
   ktimer_begin();
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, rt().stream, g);
@@ -426,7 +426,7 @@ static int gram_sets_launch(GramArgs<T>& g) {
   constexpr int ROWS = 64 / (KC / 2);
   g.ntiles = (g.nrows + 4 * ROWS - 1) / (4 * ROWS);
   const size_t lds = sizeof(T) * ((size_t)(kBlock / 64) * 3 * 256 + KC * KC);
-  const int grid = persistent_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
+  const int grid = reducing_blocks(kern, lds, g.ntiles, rt().gram_blocks_per_cu);
   g.partials = (T*)device_work(sizeof(T) * (size_t)grid * KC * KC);
   ktimer_begin();
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, rt().stream, g);
@@ -934,7 +934,7 @@ int mix_gram_launch(MixArgs<T>& p) {
   p.ntiles = (p.nrows + 64 * RT - 1) / (64 * RT);
   const int na = GRAM == 1 ? p.m : p.ngv;
   const size_t lds = sizeof(T) * na * p.m;
-  const int grid = persistent_blocks(kern, lds, p.ntiles, rt().gram_blocks_per_cu);
+  const int grid = reducing_blocks(kern, lds, p.ntiles, rt().gram_blocks_per_cu);
   p.partials = (T*)device_work(sizeof(T) * (size_t)grid * na * p.m);
   ktimer_begin();
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), lds, rt().stream, p);

@@ -605,3 +605,28 @@ def test_wide_against_narrow(be64, be32, wide, dtype):
         wb.delete()
     vb.delete()
     m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 63, 1025, 20011, 300001])
+def test_reductions_by_width(be64, be32, n, dtype):
+    """dots, norms and Gram matrices over the widths of the second reduction
+    stage (powers of two, between them, past 16 outputs), from one row to many
+    workgroups of partial sums, against FP64 sums"""
+    be = be64 if dtype == np.float64 else be32
+    eps = np.finfo(dtype).eps
+    m = be.map(n)
+    rng = np.random.default_rng(n)
+    for k in (1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 33):
+        X, Y = (rng.uniform(-1, 1, (n, k)).astype(dtype) for _ in range(2))
+        x, y = be.mvec(m, k, X), be.mvec(m, k, Y)
+        Xd, Yd = X.astype(float), Y.astype(float)
+        assert np.all(np.abs(be.dot(x, y) - (Xd * Yd).sum(0)) <= (n + 2) * eps * np.abs(Xd * Yd).sum(0)), k
+        want = np.linalg.norm(Xd, axis=0)
+        assert np.all(np.abs(be.norm2(x) - want) <= (n + 2) * eps * want), k
+        C = be.sdmat(k, k)
+        be.gram(1.0, x, y, 0.0, C)
+        assert np.all(np.abs(C.get() - Xd.T @ Yd) <= (n + 2) * eps * (np.abs(Xd).T @ np.abs(Yd))), k
+        for o in (x, y, C):
+            o.delete()
+    m.delete()
