@@ -51,11 +51,12 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
   if (Q && Q->nvec == 0) Q = nullptr;
   // the projected operator P (A + s I) with P = I - QQ' (the correction equations of
   // Jacobi-Davidson, phist_jadaOp_def.hpp:192-268): w -= Q (Q'w) after every product
+  std::unique_ptr<SdBox<TI>> qw;  // Q'w
   auto project = [&](Mvec<TI>* w) {
     if (!Q) return;
-    SdBox<TI> C(Q->nvec, w->nvec);
-    gemm_gram<TI>(TI(1), Q, w, TI(0), C.get(), false);
-    gemm_times_sd<TI>(TI(-1), Q, C.get(), TI(1), w);
+    if (!qw || qw->get()->ncols != w->nvec) qw.reset(new SdBox<TI>(Q->nvec, w->nvec));
+    gemm_gram<TI>(TI(1), Q, w, TI(0), qw->get(), false);
+    gemm_times_sd<TI>(TI(-1), Q, qw->get(), TI(1), w);
   };
   PHX_REQUIRE(m >= 1 && m <= 256, PHIST_INVALID_INPUT, "GMRES basis size %d (1..256)", m);
   PHX_REQUIRE((int64_t)(m + 1) * k <= 4096, PHIST_INVALID_INPUT, "GMRES basis (m+1)*k = %d columns too wide",
@@ -63,7 +64,10 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
   const double eps = std::numeric_limits<double>::epsilon();
   // working precision copies of b and x (all systems); the cycles run on
   // compact blocks of the systems still iterating (act: their indices)
-  MvBox<TI> b(map, k), x(map, k);
+  // (blocks that are written whole before they are read are not zeroed first; a user's operator may
+  // read its result block although beta is 0, so it gets zeroed ones)
+  const bool zero = op.user != nullptr;
+  MvBox<TI> b(map, k, false), x(map, k, false);
   copy_any<T, TI>(B, b.get());
   copy_any<T, TI>(X, x.get());
 
@@ -82,7 +86,8 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
       blas_copy<TI>(from.get(), to.get());
     }
   };
-  std::unique_ptr<MvBox<TI>> bc(new MvBox<TI>(map, k)), xc(new MvBox<TI>(map, k)), wc(new MvBox<TI>(map, k));
+  std::unique_ptr<MvBox<TI>> bc(new MvBox<TI>(map, k, false)), xc(new MvBox<TI>(map, k, false)),
+      wc(new MvBox<TI>(map, k, zero));
   blas_copy<TI>(b.get(), bc->get());
   blas_copy<TI>(x.get(), xc->get());
   std::vector<TI> s(shifts.begin(), shifts.end());
@@ -124,13 +129,18 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
         }
         done.push_back(a);
       }
+      if (keep.empty() && kk == k) {  // all at once, in their order
+        blas_copy<TI>(xc->get(), x.get());
+        break;
+      }
       for (int a : done) {
         View<TI> from(xc->get(), a, a), to(x.get(), act[a], act[a]);
         blas_copy<TI>(from.get(), to.get());
       }
       if (keep.empty()) break;
       const int kn = (int)keep.size();
-      std::unique_ptr<MvBox<TI>> bn(new MvBox<TI>(map, kn)), xn(new MvBox<TI>(map, kn)), wn(new MvBox<TI>(map, kn));
+      std::unique_ptr<MvBox<TI>> bn(new MvBox<TI>(map, kn, false)), xn(new MvBox<TI>(map, kn, false)),
+          wn(new MvBox<TI>(map, kn, false));
       cols(bc->get(), keep, bn->get());
       cols(xc->get(), keep, xn->get());
       cols(wc->get(), keep, wn->get());
@@ -155,7 +165,7 @@ GmresOut gmres_solve(const Operator<TI>& op, const std::vector<T>& shifts, const
     // vcur: the current basis vectors as a compact block (row stride kk), the
     // SpMV's input; gathering them from the side-by-side basis (row stride
     // (m+1)*kk) would fetch a cache line per entry for a few bytes of it
-    MvBox<TI> w(map, kk), Vb(map, (m + 1) * kk), vcur(map, kk);
+    MvBox<TI> w(map, kk, zero), Vb(map, (m + 1) * kk, zero), vcur(map, kk, zero);
     std::vector<double> H((size_t)kk * (m + 1) * m), cs((size_t)kk * m), sn((size_t)kk * m), g((size_t)kk * (m + 1));
     auto h = [&](int a, int r, int c) -> double& { return H[((size_t)a * m + c) * (m + 1) + r]; };
     std::vector<TI> sc(kk);

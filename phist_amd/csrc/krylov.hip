@@ -624,7 +624,23 @@ struct CgsArgs {
   T* partials;
 };
 
-template <typename T, int LMAX, int MODE>
+// A basis larger than the last-level cache is read with non-temporal loads
+// (NT): it comes from HBM in every sweep, and the blocks it would displace are
+// read again (2.1 M rows, 16 systems, 25..28 vectors, FP64: mode 4 1487 ->
+// 1410 us, k_gmres_fix_dots 1566 -> 1502 us, 5.4 TB/s; more or fewer
+// workgroups per CU change nothing).  A smaller one stays cached.
+constexpr int64_t kBasisNtBytes = int64_t(256) << 20;
+
+template <typename T, bool NT>
+__device__ inline T basis_load(__amdgpu_buffer_rsrc_t rs, int vo, int so) {
+  constexpr int aux = NT ? 2 : 0;
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, aux));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, aux));
+}
+
+template <typename T, int LMAX, int MODE, bool NT>
 __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
   extern __shared__ unsigned char cgs_lds[];
   T* sh = reinterpret_cast<T*>(cgs_lds);
@@ -659,11 +675,7 @@ __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
     T vv[LMAX];
 #pragma unroll
     for (int l = 0; l < LMAX; l++) {
-      const int so = (l < p.nl ? l : p.nl - 1) * p.kk * (int)sizeof(T);
-      if constexpr (sizeof(T) == 8)
-        vv[l] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0));
-      else
-        vv[l] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0));
+      vv[l] = basis_load<T, NT>(rs, vo, (l < p.nl ? l : p.nl - 1) * p.kk * (int)sizeof(T));
     }
     T* wr = p.w + r * p.ldw + a;
     T s = *wr;
@@ -720,7 +732,11 @@ __global__ void __launch_bounds__(kBlock) k_gmres_cgs(const CgsArgs<T> p) {
 
 template <typename T, int LMAX, int MODE>
 static void cgs_launch(CgsArgs<T> p, int grid, size_t lds) {
-  hipLaunchKernelGGL((k_gmres_cgs<T, LMAX, MODE>), dim3(grid), dim3(kBlock), lds, rt().stream, p);
+  constexpr bool LARGE = MODE == 4;  // (the sweeps of every step on a matrix of this library)
+  if (LARGE && p.nrows * p.nl * p.kk * (int64_t)sizeof(T) > kBasisNtBytes)
+    hipLaunchKernelGGL((k_gmres_cgs<T, LMAX, MODE, LARGE>), dim3(grid), dim3(kBlock), lds, rt().stream, p);
+  else
+    hipLaunchKernelGGL((k_gmres_cgs<T, LMAX, MODE, false>), dim3(grid), dim3(kBlock), lds, rt().stream, p);
   PHX_HIP(hipGetLastError());
 }
 
@@ -758,7 +774,7 @@ struct FixArgs {
   T* partials;
 };
 
-template <typename T, int LMAX>
+template <typename T, int LMAX, bool NT>
 __global__ void __launch_bounds__(kBlock) k_gmres_fix_dots(const FixArgs<T> g) {
   extern __shared__ unsigned char cgs_lds[];
   T* sh = reinterpret_cast<T*>(cgs_lds);
@@ -784,11 +800,7 @@ __global__ void __launch_bounds__(kBlock) k_gmres_fix_dots(const FixArgs<T> g) {
     T vv[LMAX];
 #pragma unroll
     for (int l = 0; l < LMAX; l++) {
-      const int so = (l < g.nl ? l : g.nl - 1) * g.kk * (int)sizeof(T);
-      if constexpr (sizeof(T) == 8)
-        vv[l] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0));
-      else
-        vv[l] = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0));
+      vv[l] = basis_load<T, NT>(rs, vo, (l < g.nl ? l : g.nl - 1) * g.kk * (int)sizeof(T));
     }
     const T pv = g.p[r * g.ldp + a], w = g.w[r * g.ldw + a];
     __builtin_amdgcn_sched_barrier(0);  // every load of the row in flight together (k_gmres_cgs)
@@ -826,7 +838,7 @@ int gmres_cgs_grid(int64_t nrows, int kk) {
   int kp = 1;
   while (kp < kk) kp <<= 1;
   const int64_t ntiles = (nrows + kBlock / kp - 1) / (kBlock / kp);
-  return persistent_blocks(k_gmres_cgs<double, 32, 1>, 2 * kGmresCgsMaxNl * 64 * sizeof(double), ntiles, 4);
+  return persistent_blocks(k_gmres_cgs<double, 32, 1, false>, 2 * kGmresCgsMaxNl * 64 * sizeof(double), ntiles, 4);
 }
 
 template <typename T>
@@ -871,7 +883,10 @@ void gmres_cgs_dev(int mode, int64_t nrows, const T* v, int64_t ldv, T* w, int64
 template <typename T, int LMAX>
 static void fix_launch(const FixArgs<T>& g, int grid) {
   const size_t lds = sizeof(T) * ((size_t)(g.nl + 1) * g.kk + (size_t)LMAX * g.kk);
-  hipLaunchKernelGGL((k_gmres_fix_dots<T, LMAX>), dim3(grid), dim3(kBlock), lds, rt().stream, g);
+  if (g.nrows * g.nl * g.kk * (int64_t)sizeof(T) > kBasisNtBytes)
+    hipLaunchKernelGGL((k_gmres_fix_dots<T, LMAX, true>), dim3(grid), dim3(kBlock), lds, rt().stream, g);
+  else
+    hipLaunchKernelGGL((k_gmres_fix_dots<T, LMAX, false>), dim3(grid), dim3(kBlock), lds, rt().stream, g);
   PHX_HIP(hipGetLastError());
 }
 

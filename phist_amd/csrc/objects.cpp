@@ -30,7 +30,7 @@ T* Mvec<T>::host() {
 namespace api {
 
 template <typename T>
-Mvec<T>* mvec_create(const Map* map, int nvec) {
+Mvec<T>* mvec_create(const Map* map, int nvec, bool zero) {
   ensure_init();
   PHX_REQUIRE(map, PHIST_INVALID_INPUT, "NULL map");
   PHX_REQUIRE(nvec > 0, PHIST_INVALID_INPUT, "mvec needs at least one column (got %d)", nvec);
@@ -46,7 +46,7 @@ Mvec<T>* mvec_create(const Map* map, int nvec) {
     delete V;
     throw;
   }
-  PHX_HIP(hipMemsetAsync(V->dev_base, 0, bytes, rt().stream));
+  if (zero) PHX_HIP(hipMemsetAsync(V->dev_base, 0, bytes, rt().stream));
   return V;
 }
 
@@ -513,7 +513,7 @@ void sdMat_add(T alpha, const SdMat<T>* A, bool ta, T beta, SdMat<T>* B) {
   template void sd_from_device<T>(const SdMat<T>*);                                      \
   template void sd_from_device_async<T>(const SdMat<T>*);                                \
   namespace api {                                                                        \
-  template Mvec<T>* mvec_create<T>(const Map*, int);                                     \
+  template Mvec<T>* mvec_create<T>(const Map*, int, bool);                               \
   template void mvec_delete<T>(Mvec<T>*);                                                \
   template void mvec_view_block<T>(Mvec<T>*, Mvec<T>**, int, int);                       \
   template void mvec_get_block<T>(const Mvec<T>*, Mvec<T>*, int, int);                   \

@@ -13,7 +13,7 @@ SparseMat<T>* sparse_from_mm(const Comm* comm, const char* filename);
 
 namespace api {
 
-template <typename T> Mvec<T>* mvec_create(const Map* map, int nvec);
+template <typename T> Mvec<T>* mvec_create(const Map* map, int nvec, bool zero = true);
 template <typename T> void mvec_delete(Mvec<T>* V);
 template <typename T> void mvec_view_block(Mvec<T>* V, Mvec<T>** Vblock, int jmin, int jmax);
 template <typename T> void mvec_get_block(const Mvec<T>* V, Mvec<T>* B, int jmin, int jmax);

@@ -58,7 +58,8 @@ template <typename T>
 struct MvBox {
   Mvec<T>* p = nullptr;
   MvBox() = default;
-  MvBox(const Map* map, int nvec) : p(api::mvec_create<T>(map, nvec)) {}
+  // zero = false: the caller writes every entry before one is read
+  MvBox(const Map* map, int nvec, bool zero = true) : p(api::mvec_create<T>(map, nvec, zero)) {}
   ~MvBox() {
     try {
       if (p) api::mvec_delete(p);
