@@ -170,34 +170,27 @@ __device__ inline void block_tile_sum(T* sh, int nout, T* __restrict__ out, F&& 
   for (int o = threadIdx.x; o < nout; o += kBlock) out[o] = sh[o];
 }
 
-// Sum over b of partials[b*width + o] for the outputs o = 16*group + i of this
-// workgroup (i < 16, returned on thread i; others get 0; every thread must
-// call it).  All threads add whatever the width: with W the power of two that
-// holds the outputs (at most 16), thread t takes output t % W and blocks b =
-// t/W, t/W + 256/W, ... in order; then the lanes of a wave that share an
-// output by shuffles and the four waves in order.  (The second stage of a
-// reduction is one workgroup's serial chain: 2048 partials of 4 columns took
-// 8.0 us with 16 lanes per column, 1024 take 3.9 us with 64.)
+// Sum over b of partials[b*width + o] for the 16 outputs o = 16*blockIdx.x +
+// (tid & 15) of this workgroup: thread group p = tid / 16 adds b = p, p+16, ...
+// in order, then the 16 group sums are added in order of p.  The result is
+// returned on threads 0..15 (others get 0); every thread must call it.  The
+// order does not depend on the width, so a column's sum over the same partials
+// is the same in blocks of any width.
 template <typename T>
 __device__ inline T block_sum16(const T* __restrict__ partials, int nblocks, int width, int group) {
-  __shared__ T sh[kBlock / 64][16];
-  const int n = min(16, width - group * 16);
-  int W = 1;
-  while (W < n) W <<= 1;
-  const int i = threadIdx.x & (W - 1), step = kBlock / W;
+  __shared__ T sh[16][17];
+  const int o = group * 16 + (threadIdx.x & 15), grp = threadIdx.x >> 4;
   T s = T(0);
-  if (i < n) {
-    const T* p = partials + group * 16 + i;
+  if (o < width) {
 #pragma unroll 8
-    for (int b = threadIdx.x / W; b < nblocks; b += step) s += p[(int64_t)b * width];
+    for (int b = grp; b < nblocks; b += kBlock / 16) s += partials[(int64_t)b * width + o];
   }
-  for (int off = W; off < 64; off <<= 1) s += __shfl_xor(s, off, 64);
-  if ((threadIdx.x & 63) < (unsigned)W) sh[threadIdx.x >> 6][i] = s;
+  sh[grp][threadIdx.x & 15] = s;
   __syncthreads();
   T t = T(0);
-  if ((int)threadIdx.x < n)
+  if (threadIdx.x < 16)
 #pragma unroll
-    for (int q = 0; q < kBlock / 64; q++) t += sh[q][threadIdx.x];
+    for (int q = 0; q < kBlock / 16; q++) t += sh[q][threadIdx.x];
   __syncthreads();  // sh may be reused by the next call
   return t;
 }

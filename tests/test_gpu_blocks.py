@@ -610,9 +610,9 @@ def test_wide_against_narrow(be64, be32, wide, dtype):
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("n", [1, 63, 1025, 20011, 300001])
 def test_reductions_by_width(be64, be32, n, dtype):
-    """dots, norms and Gram matrices over the widths of the second reduction
-    stage (powers of two, between them, past 16 outputs), from one row to many
-    workgroups of partial sums, against FP64 sums"""
+    """dots, norms and Gram matrices over widths within and past the 16 outputs
+    of a second-stage workgroup, from one row to many workgroups of partial
+    sums, against FP64 sums"""
     be = be64 if dtype == np.float64 else be32
     eps = np.finfo(dtype).eps
     m = be.map(n)
