@@ -39,6 +39,7 @@ enum : int { B_READX = 1, B_READY = 2 };
 
 // rows per lane group and tile
 constexpr int kRowUnroll = 4;
+static_assert(kRowUnroll == 4, "k_coldot adds four row sums");
 // workgroups per CU of the dots: with four rows under way per lane group four
 // keep HBM busy, and the partial sums are half as many as with eight
 constexpr int kDotBlocksPerCu = 4;
@@ -121,9 +122,12 @@ __global__ void __launch_bounds__(kBlock) k_coldot(const RowArgs<T> p) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int q = lane % LPR, rw = lane / LPR, c0 = q * VPL;
   const bool colok = c0 < p.ncols;
-  T acc[VPL];
+  // a sum for each of a tile's rows: the chains, and with them the rounding, stay as short as with a row per tile
+  T acc[kRowUnroll][VPL];
 #pragma unroll
-  for (int e = 0; e < VPL; e++) acc[e] = T(0);
+  for (int u = 0; u < kRowUnroll; u++)
+#pragma unroll
+    for (int e = 0; e < VPL; e++) acc[u][e] = T(0);
   const bool self = p.x == p.y && p.ldx == p.ldy;  // a norm reads its block once
   const TileWalk tw = xcd_tiles(p.ntiles);
   for (int64_t t = tw.t; t < tw.end; t += tw.stride) {
@@ -141,14 +145,15 @@ __global__ void __launch_bounds__(kBlock) k_coldot(const RowArgs<T> p) {
 #pragma unroll
     for (int u = 0; u < kRowUnroll; u++)
 #pragma unroll
-      for (int e = 0; e < VPL; e++) acc[e] = fma(xv[u][e], self ? xv[u][e] : yv[u][e], acc[e]);
+      for (int e = 0; e < VPL; e++) acc[u][e] = fma(xv[u][e], self ? xv[u][e] : yv[u][e], acc[u][e]);
   }
   __shared__ T red[kBlock / 64][64 * VPL];
 #pragma unroll
-  for (int e = 0; e < VPL; e++) acc[e] = wave_sum_strided<LPR>(acc[e]);
+  for (int e = 0; e < VPL; e++)
+    acc[0][e] = wave_sum_strided<LPR>((acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]));
   if (lane < LPR) {
 #pragma unroll
-    for (int e = 0; e < VPL; e++) red[wv][lane * VPL + e] = acc[e];
+    for (int e = 0; e < VPL; e++) red[wv][lane * VPL + e] = acc[0][e];
   }
   __syncthreads();
   for (int c = threadIdx.x; c < p.ncols; c += kBlock) {

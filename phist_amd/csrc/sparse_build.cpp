@@ -169,7 +169,7 @@ void sell_build(SparseMat<T>* A, int C, int sigma) {
   A->perm_identity = ident;
   double dist = 0.0;
   int64_t sampled = 0;
-  for (int64_t i = 0; i < n; i += std::max<int64_t>(1, n / 4096))
+  for (int64_t i = 0; i < n; i += std::max<int64_t>(1, n / 256))
     for (int64_t p = A->crs_ptr[i]; p < A->crs_ptr[i + 1]; p++, sampled++)
       dist += (double)std::llabs((long long)A->crs_col[p] - (long long)i);
   A->gather_span = sampled ? dist / (double)sampled : 0.0;
