@@ -23,6 +23,9 @@
 
 namespace phx {
 
+// block columns of a launch at most: the shifts that travel with its arguments
+constexpr int kSpmvMaxCols = 256;
+
 template <typename T>
 struct SpmvArgs {
   const int64_t* __restrict__ chunk_ptr;
@@ -58,7 +61,7 @@ struct SpmvArgs {
   const uint16_t* __restrict__ st_lcol;
   int st_ppr, st_pshift;
   size_t st_lds_bytes;  // host side: dynamic LDS of the staged window
-  T shift[64 * 4];
+  T shift[kSpmvMaxCols];
 };
 
 // Workgroups per CU of the staged and Gram kernels by row length and block
@@ -765,9 +768,12 @@ int launch_vpl(SpmvArgs<T>& a, int lpr, int depth) {
     case 4: return launch_rows<T, VPL, 4, 8>(a);
     case 8: return launch_rows<T, VPL, 8, 8>(a);
     case 16: return launch_rows<T, VPL, 16, 16>(a);
-    case 32: return launch_rows<T, VPL, 32, 32>(a);
-    default: return launch_rows<T, VPL, 64, 64>(a);
   }
+  if constexpr (VPL * 32 <= kSpmvMaxCols)
+    if (lpr == 32) return launch_rows<T, VPL, 32, 32>(a);
+  if constexpr (VPL * 64 <= kSpmvMaxCols)
+    if (lpr == 64) return launch_rows<T, VPL, 64, 64>(a);
+  fail(PHIST_FUNCTIONAL_ERROR, "%d lanes of %d columns in a launch", lpr, VPL);
 }
 
 template <typename T, int VPL, int LPR, int GR, int SL, bool STG>
@@ -960,12 +966,14 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   if (stage < 0) stage = rt().spmv_stage;
   if (stage < 0) stage = preset.stage;
   // block columns per lane, the gathered bytes per lane and nonzero, and per
-  // launch: 64 lane groups, or fewer as set or tuned (each further launch
-  // reads the matrix again); each row's sum is the same whichever is taken.
+  // launch: 64 lane groups and kSpmvMaxCols columns, or fewer as set or tuned
+  // (each further launch reads the matrix again); each row's sum is the same
+  // whichever is taken.
   // x rows are addressed by 32-bit byte offsets from the block's first row;
   // larger blocks (x64) take one vector per lane.
   const bool x64 = !gram && (uint64_t)x->nrows * (uint64_t)x->lda * sizeof(T) > UINT32_MAX;
   const bool tuned = tuned_at != A->tuned.end();
+  static_assert(kSpmvMaxCols % (4 * V16) == 0, "launches of whole lanes");
   int VPL = 1, maxcols = 64;
   auto shape = [&](bool with_preset) {
     int lb = rt().spmv_lane_bytes, colblock = req.col_block;
@@ -974,13 +982,13 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
     if (colblock < 0) colblock = rt().spmv_col_block;
     if (colblock < 0) colblock = with_preset ? preset.col_block : 0;
     VPL = spmv_lane_columns<T>(nvec, x64 && lb > 16 ? 0 : lb);
-    maxcols = 64 * VPL;
+    maxcols = std::min(64 * VPL, kSpmvMaxCols);
     if (colblock > 0 && colblock % VPL == 0) maxcols = std::min(maxcols, colblock);
   };
   bool staged = false;
   if (gram) {
     VPL = vec_ok ? V16 : 1;
-    maxcols = 64 * VPL;
+    maxcols = std::min(64 * VPL, kSpmvMaxCols);
   } else {
     // staging forced on or off keeps the 16-byte lanes either way, so that both products' dots group alike
     shape(tuned || (req.stage < 0 && rt().spmv_stage < 0));

@@ -7,6 +7,7 @@ Bars: index work (CRS order, SELL layout) bit-exact; FP64 results within
 1e-5 relative to the FP64 oracle.  The reference's own golden vectors
 (A2_precalc_result) are checked to sqrt(eps) as in its test.
 """
+import ctypes
 import json
 import os
 
@@ -581,4 +582,55 @@ def test_spmv_block_over_4_gib(be64, k):
     assert np.array_equal(y.get(), want)
     for o in (xv, wide, x, y, A):
         o.delete()
+    m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["sheet", "stencil", "band12", "band30"])
+def test_spmv_blocks_past_one_launch(be64, be32, kind, dtype):
+    """blocks wider than the 256 columns of a launch, at every lane width: the
+    columns equal those of products of at most 100 columns bit for bit, plain
+    and with a shift per column, and the dots agree with the columns"""
+    be = be64 if dtype == np.float64 else be32
+    A = {"sheet": lambda: be.honeycomb(19, 23, 0, 0, 0, 1.0, 7), "stencil": lambda: be.laplace3d(9, 7, 8),
+         "band12": lambda: be.banded_random(501, 12, 60, 40.0, 5),
+         "band30": lambda: be.banded_random(497, 30, 100, 40.0, 6)}[kind]()
+    n, widest = A.nrows, 1048
+    rng = np.random.default_rng(23)
+    X, Y0 = (rng.uniform(-1, 1, (n, widest)).astype(dtype) for _ in range(2))
+    sh = rng.uniform(-2, 2, widest).astype(dtype)
+    m = be.map(n)
+    one, shifted = np.empty_like(X), np.empty_like(X)
+    for c in range(0, widest, 100):
+        s = slice(c, min(widest, c + 100))
+        x, y = be.mvec(m, s.stop - c, X[:, s]), be.mvec(m, s.stop - c)
+        be.spmv(0.75, A, x, 0.0, y)
+        one[:, s] = y.get()
+        y.set(Y0[:, s])
+        be.spmv_shifted(0.75, A, sh[s], x, -0.3, y)
+        shifted[:, s] = y.get()
+        x.delete()
+        y.delete()
+    tol = 1e-12 if dtype == np.float64 else 1e-4  # sums of at most 504 products
+    fl = ctypes.c_int(0)
+    try:
+        for lane_bytes in (0, np.dtype(dtype).itemsize, 32, 64):
+            be.L.phist_amd_set_spmv_lane_bytes(lane_bytes, ctypes.byref(fl))
+            assert fl.value == 0
+            for k in (255, 256, 257, 264, 272, 511, 512, 520, 1024, 1048):
+                x, y = be.mvec(m, k, X[:, :k]), be.mvec(m, k, Y0[:, :k])
+                be.spmv_shifted(0.75, A, sh[:k], x, -0.3, y)
+                assert np.array_equal(y.get(), shifted[:, :k]), (lane_bytes, k)
+                be.spmv(0.75, A, x, 0.0, y)
+                assert np.array_equal(y.get(), one[:, :k]), (lane_bytes, k)
+                ww, vw = be.fused_spmv_mvdot(0.75, A, x, 0.0, y)
+                assert np.array_equal(y.get(), one[:, :k]), (lane_bytes, k)
+                w, v = one[:, :k].astype(float), X[:, :k].astype(float)
+                assert np.all(np.abs(ww - (w * w).sum(0)) <= tol * (w * w).sum(0)), (lane_bytes, k)
+                assert np.all(np.abs(vw - (v * w).sum(0)) <= tol * np.abs(v * w).sum(0)), (lane_bytes, k)
+                x.delete()
+                y.delete()
+    finally:
+        be.L.phist_amd_set_spmv_lane_bytes(0, ctypes.byref(fl))
+    A.delete()
     m.delete()
