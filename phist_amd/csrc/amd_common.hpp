@@ -390,6 +390,7 @@ struct SparseMat {
   T* d_val = nullptr;              // [nnz_padded] value of each slot
   bool perm_identity = true;
   double gather_span = 0.0;  // mean distance of a sample of the entries from the diagonal (rows)
+  double gather_next = 0.0;  // share of the sample whose next row has an entry in the next column
   // host copies of the SELL index arrays (for inspection)
   std::vector<int64_t> h_chunk_ptr;
   std::vector<int32_t> h_chunk_w;

@@ -168,11 +168,18 @@ void sell_build(SparseMat<T>* A, int C, int sigma) {
   A->nnz_padded = nslot_el;
   A->perm_identity = ident;
   double dist = 0.0;
-  int64_t sampled = 0;
-  for (int64_t i = 0; i < n; i += std::max<int64_t>(1, n / 256))
-    for (int64_t p = A->crs_ptr[i]; p < A->crs_ptr[i + 1]; p++, sampled++)
+  int64_t sampled = 0, next = 0;
+  for (int64_t i = 0; i < n; i += std::max<int64_t>(1, n / 256)) {
+    int64_t q = i + 1 < n ? A->crs_ptr[i + 1] : 0;
+    const int64_t qend = i + 1 < n ? A->crs_ptr[i + 2] : 0;
+    for (int64_t p = A->crs_ptr[i]; p < A->crs_ptr[i + 1]; p++, sampled++) {
       dist += (double)std::llabs((long long)A->crs_col[p] - (long long)i);
+      while (q < qend && A->crs_col[q] <= A->crs_col[p]) q++;  // both rows are sorted
+      next += q < qend && A->crs_col[q] == A->crs_col[p] + 1;
+    }
+  }
   A->gather_span = sampled ? dist / (double)sampled : 0.0;
+  A->gather_next = sampled ? (double)next / (double)sampled : 0.0;
   hipStream_t st = r.stream;
   PHX_HIP(hipMalloc(&A->d_chunk_ptr, (nchunks + 1) * sizeof(int64_t)));
   PHX_HIP(hipMalloc(&A->d_chunk_w, std::max<int64_t>(1, nchunks) * sizeof(int32_t)));

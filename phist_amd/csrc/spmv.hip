@@ -20,6 +20,7 @@
 // workgroup through LDS, and across workgroups by a second fixed-order pass.
 #include "amd_device.hpp"
 #include <algorithm>
+#include <type_traits>
 
 namespace phx {
 
@@ -44,7 +45,8 @@ struct SpmvArgs {
   int64_t ldu;
   int ncols;  // block columns handled by this launch
   bool x64;   // host side: x offsets need 64 bits
-  bool full;  // host side: the instance with epilogues
+  bool full;   // host side: the instance with epilogues
+  bool ahead;  // host side: its gathers under way together (AHEAD)
   int nact;   // lanes of columns >= nact skip their loads and stores (same kernel, grid and sums)
   T alpha, beta, gamma, delta;
   int flags;
@@ -163,7 +165,17 @@ __device__ inline T group_bcast_t(T v, int src, int lane) {
 // rows x 32 in a band of +-50k, 8 columns 1242 -> 1001, 32 columns 4962 ->
 // 3280 (floors by the byte model at 5.5 TB/s: 35, 815, 68, 86, 38, 129, 390
 // and 683).
-template <typename T, int VPL, int LPR, int SL, bool FULL, bool X64>
+//
+// AHEAD: the x offsets of a batch are settled before its first gather.
+// Without it the compiler of the epilogue instance forms each offset in a
+// register of that gather's result and has every gather wait for those before
+// it.  That pacing suits long rows whose x lines miss the L1 and evict each
+// other there, but where neighbouring rows gather neighbouring x rows, or few
+// waves run, it leaves the latency uncovered (shifted products of 64-byte x
+// rows, FP64 / FP32, us: 22-spin chain 95 / 97 paced, 79 / 72 together; 100^3
+// Laplacian 68 / 62, 55 / 51; 4000 rows x 32: 7.7 / 7.3, 6.4 / 6.1; but 600 k
+// x 20 in +-2000: 91 / 84, 109 / 98).
+template <typename T, int VPL, int LPR, int SL, bool FULL, bool X64, bool AHEAD = false>
 __global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
   constexpr int RPW = 64 / LPR;
   constexpr int RPB = (kBlock / 64) * RPW;
@@ -186,13 +198,12 @@ __global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
     sh[e] = (colok && (flags & F_SHIFT)) ? (a.shift_dev ? a.shift_dev[c0 + e] : a.shift[c0 + e]) : T(0);
     dww[e] = dvw[e] = T(0);
   }
-  // x row of column cc: byte offsets of 32 bits from a.x unless the block is larger (X64)
-  const uint32_t xld = (uint32_t)(a.ldx * (int64_t)sizeof(T)), xc0 = (uint32_t)c0 * (uint32_t)sizeof(T);
-  auto gather = [&](int32_t cc, T (&out)[VPL]) {
-    if constexpr (X64)
-      uload<T, VPL>(a.x + (int64_t)cc * a.ldx + c0, out);
-    else
-      uload<T, VPL>(reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.x) + ((uint32_t)cc * xld + xc0)), out);
+  // byte offset of x row cc from a.x, of 32 bits unless the block is larger (X64)
+  using off_t = std::conditional_t<X64, int64_t, uint32_t>;
+  const off_t xld = (off_t)(a.ldx * (int64_t)sizeof(T)), xc0 = (off_t)(c0 * (int)sizeof(T));
+  auto offset = [&](int32_t cc) { return (off_t)cc * xld + xc0; };
+  auto gather = [&](off_t o, T (&out)[VPL]) {
+    uload<T, VPL>(reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.x) + o), out);
   };
 
   // a row's chunk width and the slot of its first entry, from the first slot
@@ -249,7 +260,7 @@ __global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
     T acc[VPL], xo[VPL], yo[VPL];
 #pragma unroll
     for (int e = 0; e < VPL; e++) xo[e] = yo[e] = T(0);
-    if (FULL && live && (flags & (F_SHIFT | F_DVW))) gather(row, xo);
+    if (FULL && live && (flags & (F_SHIFT | F_DVW))) gather(offset(row), xo);
     if (FULL && live && (flags & F_BETA)) uload<T, VPL>(a.y + (int64_t)row * a.ldy + c0, yo);
 #pragma unroll
     for (int e = 0; e < VPL; e++) acc[e] = (flags & F_SHIFT) ? sh[e] * xo[e] : T(0);
@@ -257,18 +268,27 @@ __global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
     load_batch(cur, 0, v, cj);
     for (int j0 = 0; __any(j0 < cur.w);) {
       const bool more = __any(j0 + BATCH < cur.w);  // uniform over the wave
+      // slot j0+k of this row sits in lane k % LPR of the group, register k / LPR
+      off_t xoff[SUB];
+      if constexpr (AHEAD) {
+        static_assert(SUB == BATCH, "one set of offsets a batch");
+#pragma unroll
+        for (int k = 0; k < SUB; k++) {
+          xoff[k] = offset(group_bcast<LPR>(cj[k / LPR], k % LPR, lane));
+          asm volatile("" : "+v"(xoff[k]));  // settled here
+        }
+      }
       T vn[KB];
       int32_t cn[KB];
       if (more) load_batch(cur, j0 + BATCH, vn, cn);
-      // slot j0+k of this row sits in lane k % LPR of the group, register k / LPR
 #pragma unroll
       for (int k0 = 0; k0 < BATCH; k0 += SUB) {
         T xg[SUB][VPL];
 #pragma unroll
         for (int kk = 0; kk < SUB; kk++) {
           const int k = k0 + kk;
-          const int32_t cc = group_bcast<LPR>(cj[k / LPR], k % LPR, lane);
-          if (colok && (j0 + k) < cur.w) gather(cc, xg[kk]);
+          if constexpr (!AHEAD) xoff[kk] = offset(group_bcast<LPR>(cj[k / LPR], k % LPR, lane));
+          if (colok && (j0 + k) < cur.w) gather(xoff[kk], xg[kk]);
         }
 #pragma unroll
         for (int kk = 0; kk < SUB; kk++) {
@@ -741,6 +761,10 @@ int launch_rows(SpmvArgs<T>& a) {
   if (a.x64) {
     if constexpr (VPL * sizeof(T) <= 16) return launch_kernel(k_spmv<T, VPL, LPR, SF, true, true>, a, rows, 0);
   }
+  // (narrower lanes, single ones, wider groups and short batches of four lanes have their gathers
+  // together as it is, or gain nothing)
+  if constexpr ((LPR == 2 || (LPR == 4 && SL > 4)) && VPL * sizeof(T) == 16)
+    if (a.full && a.ahead) return launch_kernel(k_spmv<T, VPL, LPR, SF, true, false, true>, a, rows, 0);
   return a.full ? launch_kernel(k_spmv<T, VPL, LPR, SF, true, false>, a, rows, 0)
                 : launch_kernel(k_spmv<T, VPL, LPR, SL, false, false>, a, rows, 0);
 }
@@ -864,36 +888,89 @@ const SellStage* spmv_stage_for(const SparseMat<T>* A, int nc, int vpl, int* psh
 template const SellStage* spmv_stage_for<double>(const SparseMat<double>*, int, int, int*, size_t*);
 template const SellStage* spmv_stage_for<float>(const SparseMat<float>*, int, int, int*, size_t*);
 
-// rows whose products always take the instance with epilogues: it keeps
-// fewer gathers under way per wave, which long rows want (their x lines miss
-// the L1, and more lines under way than it holds evict each other; 4.2 M rows
-// x 32 in a band of +-50k, us: 8 columns 1001 against 1157, 4 columns 703 /
-// 815, 16: 1622 / 1805; 300 k x 24 in +-400, 8 columns 44 / 48)
+// long rows: at least 24 entries on average
 template <typename T>
 inline bool spmv_long_rows(const SparseMat<T>* A) {
   return A->nnz >= 24 * std::max<int64_t>(1, A->nrows);
 }
 
+// What the x rows of a product with nvec columns cost to gather, from the
+// rows' bytes and a sample of the entries.  few: the row groups leave the
+// chip at no more than two waves per SIMD, whose latency nothing covers.
+// near: neighbouring rows gather neighbouring x rows (a stencil, a chain).
+// window: bytes of x within reach of neighbouring rows; up to 16 KB (local)
+// they stay in the L1, and from 512 KB (wide) on they are a share of the L2.
+struct SpmvReach {
+  int rb;  // bytes of an x row
+  double window;
+  bool few, near, local, wide;
+  bool scattered() const { return !few && !near && !local; }
+};
+template <typename T>
+SpmvReach spmv_reach(const SparseMat<T>* A, int nvec) {
+  SpmvReach r;
+  r.rb = nvec * (int)sizeof(T);
+  int lanes = 1;
+  while (lanes * 16 < r.rb && lanes < 64) lanes <<= 1;
+  r.few = A->nrows * lanes <= (int64_t)rt().num_cu * 512;
+  r.near = A->gather_next >= 0.5;
+  r.window = 4.0 * A->gather_span * r.rb;
+  r.local = r.window <= 16.0 * 1024.0;
+  r.wide = r.window >= 512.0 * 1024.0;
+  return r;
+}
+
+// long rows of more than 128 bytes of columns: launches of 128 bytes each
+// (every launch reads the matrix again) where a launch's share of x is large
+// for the L2 or the whole block for the last-level cache, and long enough to
+// hide the further launches (FP64, us, in launches of 128 bytes / in one:
+// 600 k rows x 32 in +-50k, 32 columns 462 / 667, in +-2000 460 / 390, 150 k
+// in +-2000 106 / 87, 30 k 22 / 18, 4000 rows 17 / 6, 64 columns 33 / 7)
+inline bool spmv_col_blocks(const SpmvReach& r, int64_t nrows) {
+  const double mib = 1024.0 * 1024.0, block = (double)nrows * r.rb;
+  return r.rb > 128 && ((r.window >= 4.0 * mib && block >= 32.0 * mib) || (!r.wide && block >= 128.0 * mib));
+}
+
+// Whether a product takes the instance with epilogues (needs: it has one).
+// Plain products of long rows over scattered x rows take it as well: it keeps
+// fewer gathers under way per wave, which they want (their x lines miss the
+// L1, and more lines under way than it holds evict each other; 4.2 M rows x 32
+// in a band of +-50k, us: 8 columns 1001 against 1157, 4 columns 703 / 815,
+// 16: 1622 / 1805; 300 k x 24 in +-400, 8 columns 44 / 48), unless one launch
+// covers more than 128 bytes of columns (600 k x 32 in +-2000, 32 columns 449
+// against 390).
+template <typename T>
+bool spmv_full_instance(const SparseMat<T>* A, const SpmvReach& r, bool needs) {
+  return needs ||
+         (spmv_long_rows(A) && r.scattered() && (r.rb <= 128 || spmv_col_blocks(r, A->ncols)));
+}
+
 // Launch of k_spmv for a matrix without settings, from sweeps over lane
 // widths, depths, workgroups per CU and column blocks (us; "b" = workgroups
-// per CU; plain / shifted = the two instances):
+// per CU; plain / shifted = without / with an epilogue):
 //  - long rows: depth 8; x rows of 128 bytes and more in 32-byte lanes (16
-//    columns 1622 against 1987 and more), wider blocks in launches of 128
-//    bytes (32 columns: 3280 against 4550); where the columns of neighbouring
-//    rows span more of x than a share of the L2 (512 KB), narrow x rows want
-//    few workgroups (+-50k, 1 column: 788 at b1, 880 from b3; 4 columns: 703
-//    at b3, 790 from b4)
+//    columns 1622 against 1987 and more), wider blocks as spmv_col_blocks;
+//    where the columns of neighbouring rows span more of x than a share of
+//    the L2 (512 KB), narrow x rows want few workgroups (+-50k, 1 column: 788
+//    at b1, 880 from b3; 4 columns: 703 at b3, 790 from b4), and so does one
+//    launch of a wide block (600 k in +-2000, 64 columns shifted: 732 at b2,
+//    793 in launches of 16); few waves want short chains instead: 16-byte
+//    lanes, depth 16 (4000 rows, 16 columns: 6.3 against 8.6 in 32-byte lanes)
 //  - rows of 9 to 23 entries, plain: depth 16 (24-spin chain, 4 columns: FP64
 //    177 against 191 at depth 8, FP32 106 / 112; graphene, 8 columns 80 /
 //    80), 32-byte lanes for x rows of 128 bytes (16 columns: 528 against
-//    600); shifted: depth 8, x rows of 32 bytes gathered over a wide span in
-//    one lane (chain, 4 columns: 190 at b2, 256 in two lanes; 1 M x 12 in
-//    +-3000: 93 in one, 70 in two), from 128 bytes on b4 (601 / 629)
+//    600); shifted: depth 8, x rows of 128 bytes and more in 32-byte lanes, b4
+//    (16 columns, graphene of 700 x 701: 64 against 73 in 16-byte lanes, 600 k
+//    x 20 in +-50k 166 / 200), but for a chain's (22 spins: 150 / 136) and
+//    near-full rows' within the L1 (150 k x 20 in +-60: 35 / 33)
 //  - rows of at most 8 entries (a 3D stencil): one batch; x rows of 32 bytes
 //    in one lane (64 x 58 x 51 grid: 5.9 against 6.8, 128^3 shifted: 66 /
-//    79) unless that leaves the chip without waves (below 128 Ki rows, two
-//    per SIMD; 32^3 with dots 6.9 against 5.8), from 64 bytes on b4 (128^3, 8 columns: 106 at b4, 111 at b6; 16:
-//    213 / 219), shifted only from 128 (8 columns 143 at b4, 125 at b6)
+//    79) unless that leaves the chip without waves (below two per SIMD; 32^3
+//    with dots 6.9 against 5.8) or the x rows are scattered (600 k x 6 in
+//    +-50k: 37 in one lane, 32 in two), from 64 bytes on b4 (128^3, 8 columns:
+//    106 at b4, 111 at b6; 16: 213 / 219), shifted only from 128 (8 columns
+//    143 at b4, 125 at b6), then in 32-byte lanes for blocks the last-level cache
+//    holds (32 FP32 columns: 100^3 93 against 99, 128^3 254 against 232)
 //  - rows of at most 4 entries (a sheet): x rows of 128 bytes and more in
 //    32-byte lanes, b3 (8 M rows, 32 columns: 1092 against 1470 in 16-byte
 //    lanes; 12 columns, 96 bytes: 466 / 475), else b6 (5 columns: 45 at b6,
@@ -901,24 +978,28 @@ inline bool spmv_long_rows(const SparseMat<T>* A) {
 template <typename T>
 SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
   SpmvTuned d;
-  const int rb = nvec * (int)sizeof(T);
+  const SpmvReach r = spmv_reach(A, nvec);
+  const int rb = r.rb;
   d.blocks_per_cu = 0;
-  const bool wide = 4.0 * A->gather_span * rb >= 512.0 * 1024.0;  // the span of x that neighbouring rows read
   if (spmv_long_rows(A)) {
-    if (rb > 128) d.col_block = 128 / (int)sizeof(T);
-    d.lane_bytes = rb >= 128 ? 32 : 0;
-    if (wide && rb <= 32) d.blocks_per_cu = rb <= 8 ? 1 : 3;
+    const bool cols = spmv_col_blocks(r, A->ncols);
+    if (cols) d.col_block = 128 / (int)sizeof(T);
+    d.lane_bytes = rb >= 128 && !r.few ? 32 : 0;
+    d.depth = !r.few ? 8 : 16;
+    if (r.wide && !r.few) d.blocks_per_cu = rb <= 8 ? 1 : rb <= 32 ? 3 : rb > 128 && !cols && full ? 2 : 0;
   } else if (A->max_row_len > 8) {
     if (full) {
-      const bool far = rb == 32 && wide;
-      d.lane_bytes = far ? 32 : 0;
-      d.blocks_per_cu = far ? 2 : rb >= 128 ? 4 : 0;
+      const bool chain = r.near && r.wide, near_full = r.local && A->nnz >= 16 * A->nrows;
+      d.lane_bytes = rb >= 128 && !r.few && !chain && !near_full ? 32 : 0;
+      d.blocks_per_cu = rb >= 128 ? 4 : 0;
     } else {
       d.depth = rb > 8 ? 16 : 8;
       d.lane_bytes = rb >= 128 ? 32 : 0;
     }
   } else if (A->max_row_len > 4) {
-    d.lane_bytes = (rb == 32 && A->nrows >= (1 << 17)) || rb >= 256 ? 32 : 0;
+    const bool last_level = (double)A->nrows * rb < 128.0 * 1024.0 * 1024.0;  // x fits its share of that cache
+    const bool one_lane = rb == 32 && r.near && A->nrows >= (int64_t)rt().num_cu * 512;
+    d.lane_bytes = one_lane || rb >= 256 || (full && rb >= 128 && !r.few && last_level) ? 32 : 0;
     d.blocks_per_cu = rb >= (full ? 128 : 64) ? 4 : 6;
   } else {
     d.lane_bytes = rb >= 128 ? 32 : 0;
@@ -958,8 +1039,9 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   if (y) vec_ok = vec_ok && (y->lda % V16 == 0) && aligned16(y->dev());
   if (req.axpy_u) vec_ok = vec_ok && (U->lda % V16 == 0) && aligned16(U->dev());
   const auto tuned_at = A->tuned.find(nvec);
-  const bool full = spmv_long_rows(A) || req.has_shift || req.has_beta || req.dot_ww || req.dot_vw || req.axpy_u ||
-                    req.xscale;
+  const bool needs = req.has_shift || req.has_beta || req.dot_ww || req.dot_vw || req.axpy_u || req.xscale;
+  const SpmvReach reach = spmv_reach(A, nvec);
+  const bool full = spmv_full_instance(A, reach, needs);
   const SpmvTuned preset = tuned_at != A->tuned.end() ? tuned_at->second : spmv_default_launch(A, nvec, full);
   // x rows of each tile staged in LDS (where the matrix's tiles allow it)
   int stage = req.stage;
@@ -1008,6 +1090,7 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   a.nrows = A->nrows;
   a.x64 = x64;
   a.full = full;
+  a.ahead = !reach.scattered();
   a.nslots = A->nchunks * A->C;
   a.ldx = x->lda;
   a.ldy = y ? y->lda : 0;

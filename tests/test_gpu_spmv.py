@@ -634,3 +634,51 @@ def test_spmv_blocks_past_one_launch(be64, be32, kind, dtype):
         be.L.phist_amd_set_spmv_lane_bytes(0, ctypes.byref(fl))
     A.delete()
     m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind,widths", [("stencil", (4, 5, 8)), ("chain", (4, 7, 8)), ("band12", (4, 5, 8, 16)),
+                                         ("band30", (4, 5, 8, 33)), ("far30", (1, 33, 65)), ("short30", (4, 16, 33))])
+def test_spmv_launch_rules(be64, be32, kind, widths, dtype):
+    """the launches chosen by rows in flight, by how near and how far apart
+    the gathered x rows lie and by the size of the block: each gives the
+    columns of the one-column products bit for bit, plain and shifted with
+    beta, and dots that agree with them"""
+    be = be64 if dtype == np.float64 else be32
+    A = {"stencil": lambda: be.laplace3d(53, 52, 51), "chain": lambda: be.spinchain_sz(19, 9),
+         "band12": lambda: be.banded_random(70001, 12, 3000, 40.0, 5),
+         "band30": lambda: be.banded_random(40001, 30, 3000, 40.0, 6),
+         "far30": lambda: be.banded_random(140001, 30, 35000, 40.0, 7),
+         "short30": lambda: be.banded_random(5001, 30, 1200, 40.0, 8)}[kind]()
+    n, widest = A.nrows, max(widths)
+    rng = np.random.default_rng(29)
+    X, Y0 = (rng.uniform(-1, 1, (n, widest)).astype(dtype) for _ in range(2))
+    sh = rng.uniform(-2, 2, widest).astype(dtype)
+    m = be.map(n)
+    one, shifted = np.empty_like(X), np.empty_like(X)
+    x, y = be.mvec(m, 1), be.mvec(m, 1)
+    for c in range(widest):
+        x.set(X[:, c:c + 1])
+        be.spmv(0.75, A, x, 0.0, y)
+        one[:, c:c + 1] = y.get()
+        y.set(Y0[:, c:c + 1])
+        be.spmv_shifted(0.75, A, sh[c:c + 1], x, -0.3, y)
+        shifted[:, c:c + 1] = y.get()
+    x.delete()
+    y.delete()
+    eps = np.finfo(dtype).eps
+    for k in widths:
+        x, y = be.mvec(m, k, X[:, :k]), be.mvec(m, k, Y0[:, :k])
+        be.spmv_shifted(0.75, A, sh[:k], x, -0.3, y)
+        assert np.array_equal(y.get(), shifted[:, :k]), k
+        be.spmv(0.75, A, x, 0.0, y)
+        assert np.array_equal(y.get(), one[:, :k]), k
+        ww, vw = be.fused_spmv_mvdot(0.75, A, x, 0.0, y)
+        assert np.array_equal(y.get(), one[:, :k]), k
+        w, v = one[:, :k].astype(float), X[:, :k].astype(float)
+        assert np.all(np.abs(ww - (w * w).sum(0)) <= (n + 2) * eps * (w * w).sum(0)), k
+        assert np.all(np.abs(vw - (v * w).sum(0)) <= (n + 2) * eps * np.abs(v * w).sum(0)), k
+        x.delete()
+        y.delete()
+    A.delete()
+    m.delete()
