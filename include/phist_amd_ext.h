@@ -78,24 +78,26 @@ void phist_amd_spmv_staged_launches(int64_t* count, int* iflag);
 /* SpMV autotuner.  For each block width nvecs[0..n_nvec) (1..256, at most 16
  * widths) it times the product y = A*x on the device over the gather width
  * per lane (one scalar, or one, two or four 16-byte vectors: how many lanes
- * share a row), the workgroups per CU (1, 2, 3, 4, 6, 8), for rows of 9 to
- * 23 entries the depth (8 or 16, phist_amd_set_spmv_depth), for more
+ * share a row), the workgroups per CU (1, 2, 3, 4, 6, 8), for rows of more than
+ * 8 entries the depth (8 or 16, phist_amd_set_spmv_depth), for more
  * than 16 columns launches of 16 (and of 32 above 32) columns
  * (phist_amd_set_spmv_col_block), where the matrix allows it x staged in LDS
  * per workgroup tile (phist_amd_set_spmv_stage), and with
  * flags & 1 also over the SELL-C-sigma layout (C = 16, 32, 64; sigma = 1,
  * 256; the device copy is rebuilt from the host CRS for each).  The best
  * layout (least total time over the widths) is kept, and the best launch
- * settings of each width are stored on the matrix: later SpMVs of that width
- * use them unless phist_amd_set_spmv_lane_bytes / _blocks_per_cu / _depth / _col_block / _stage set global
- * values.  Choices are cached for the process by matrix signature (scalar
+ * settings of each width are stored on the matrix: later plain products of
+ * that width use them, and products with shifts, beta, dots or a second update
+ * settings that are found the same way with the shifted product, unless phist_amd_set_spmv_lane_bytes / _blocks_per_cu / _depth / _col_block / _stage set global
+ * values.  The library's untuned choice stays where no other is faster.
+ * Choices are cached for the process by matrix signature (scalar
  * type, rows, entries, longest row, mean distance of entries from the
  * diagonal, block width); flags & 2 measures again instead of using the
  * cache; flags & 4 (D only) also tunes the matrix's FP32 copy used by the
  * mixed-precision solvers (launch settings, same widths).  Outputs may be
  * NULL: default_ms[i] / tuned_ms[i] = fastest of three products with the
  * library's untuned choice on the incoming layout / with the chosen settings;
- * settings[7*i..7*i+6] = C, sigma, lane bytes, workgroups per CU, depth, column block,
+ * settings[7*i..7*i+6] (of the plain product) = C, sigma, lane bytes, workgroups per CU, depth, column block,
  * staging (1 = x staged in LDS).  Products
  * are identical bit for bit under every setting. */
 void phist_Damd_sparseMat_tune(phist_DsparseMat_ptr A, int n_nvec, const int* nvecs, int flags, double* default_ms,

@@ -328,9 +328,11 @@ inline int spmv_lane_columns(int nvec, int lb) {
 }
 
 // the depth the SpMV runs for a requested depth, the scalars per lane vpl,
-// the scalar size and the block width: 16 needs at most 32 gathered bytes per
-// lane and at most 8 lanes per row; otherwise 8
-inline int spmv_effective_depth(int depth, int vpl, int scalar_bytes, int ncols) {
+// the scalar size, the block width and the kernel's instance: 16 needs at
+// most 32 gathered bytes per lane, at most 8 lanes per row and the instance
+// without epilogues; otherwise 8 (less where no row is that long)
+inline int spmv_effective_depth(int depth, int vpl, int scalar_bytes, int ncols, bool full) {
+  if (full) return 8;
   int groups = (std::min(ncols, 64 * vpl) + vpl - 1) / vpl, lpr = 1;
   while (lpr < groups) lpr <<= 1;
   if (lpr > 8 || vpl * scalar_bytes > 32) return 8;
@@ -399,8 +401,9 @@ struct SparseMat {
   // use, freed with the matrix)
   SparseMat<float>* fp32_twin = nullptr;
   // SpMV launch settings the autotuner chose for this matrix, by block width
-  // (tune.cpp); the SpMV uses them unless a global setting overrides them
-  std::map<int, SpmvTuned> tuned;
+  // and whether the product has an epilogue (a shift, beta, dots, a second
+  // update; tune.cpp); the SpMV uses them unless a global setting overrides them
+  std::map<std::pair<int, bool>, SpmvTuned> tuned;
   // LDS staging tables by tile height (sell_stage; made on first use, freed
   // with the SELL copy)
   mutable std::map<int, SellStage> stage;
@@ -416,6 +419,10 @@ constexpr int kStageLdsBytes = 64 << 10;
 // the staging tables for an SpMV launch of nc columns with vpl scalars per
 // lane (spmv.hip), with log2 of the 16-byte pieces per window row and the
 // window's LDS bytes; nullptr where that launch cannot stage
+// the launch a product of nvec columns without settings takes, and whether
+// the kernel's instance with epilogues runs it
+template <typename T>
+SpmvTuned spmv_rule_launch(const SparseMat<T>* A, int nvec, bool epilogue, bool* full);
 template <typename T>
 const SellStage* spmv_stage_for(const SparseMat<T>* A, int nc, int vpl, int* pshift, size_t* lds_bytes);
 

@@ -1009,6 +1009,15 @@ SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
 }
 
 template <typename T>
+SpmvTuned spmv_rule_launch(const SparseMat<T>* A, int nvec, bool epilogue, bool* full) {
+  const bool f = spmv_full_instance(A, spmv_reach(A, nvec), epilogue);
+  if (full) *full = f;
+  return spmv_default_launch(A, nvec, f);
+}
+template SpmvTuned spmv_rule_launch<double>(const SparseMat<double>*, int, bool, bool*);
+template SpmvTuned spmv_rule_launch<float>(const SparseMat<float>*, int, bool, bool*);
+
+template <typename T>
 void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mvec<T>* x, T beta, Mvec<T>* y,
                  const SpmvRequest& req, T* dot_ww_host, T* dot_vw_host, T gamma, T delta, Mvec<T>* U) {
   const int nvec = x->nvec;
@@ -1038,10 +1047,10 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   bool vec_ok = (nvec % V16 == 0) && (x->lda % V16 == 0) && aligned16(x->dev());
   if (y) vec_ok = vec_ok && (y->lda % V16 == 0) && aligned16(y->dev());
   if (req.axpy_u) vec_ok = vec_ok && (U->lda % V16 == 0) && aligned16(U->dev());
-  const auto tuned_at = A->tuned.find(nvec);
   const bool needs = req.has_shift || req.has_beta || req.dot_ww || req.dot_vw || req.axpy_u || req.xscale;
   const SpmvReach reach = spmv_reach(A, nvec);
   const bool full = spmv_full_instance(A, reach, needs);
+  const auto tuned_at = A->tuned.find({nvec, needs});
   const SpmvTuned preset = tuned_at != A->tuned.end() ? tuned_at->second : spmv_default_launch(A, nvec, full);
   // x rows of each tile staged in LDS (where the matrix's tiles allow it)
   int stage = req.stage;
@@ -1108,7 +1117,6 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   // workgroups per CU
   int bpc = req.blocks_per_cu;
   if (bpc < 0) bpc = rt().spmv_blocks_per_cu;
-  const bool bpc_set = bpc >= 0 || tuned;
   a.blocks_per_cu = bpc >= 0 ? bpc : preset.blocks_per_cu;
   // entries per row whose loads go out together
   int depth = req.depth;
@@ -1138,11 +1146,9 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
     while (lpr < groups) lpr <<= 1;
     a.xscale = req.xscale ? req.xscale + (int64_t)cb * req.xscale_stride : nullptr;
     a.xscale_stride = req.xscale_stride;
-    const int staged_bpc =
-        bpc_set ? a.blocks_per_cu
-                : spmv_table_blocks_per_cu(A->nrows ? (double)A->nnz / (double)A->nrows : 0.0, nvec);
-    if (gram) {  // one column block (nvec <= 32)
-      a.blocks_per_cu = staged_bpc;
+    const int table_bpc = spmv_table_blocks_per_cu(A->nrows ? (double)A->nnz / (double)A->nrows : 0.0, nvec);
+    if (gram) {  // one column block (nvec <= 32); the tuner times the other kernels
+      a.blocks_per_cu = bpc >= 0 ? bpc : table_bpc;
       const int grid = vec_ok ? launch_gram<T, V16>(a, lpr) : launch_gram<T, 1>(a, lpr);
       const int nn = nc * nc;
       if (req.gram_ww_dev) {
@@ -1164,7 +1170,7 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
     int grid;
     if (S) {
       rt().spmv_staged_launches++;
-      a.blocks_per_cu = staged_bpc;
+      a.blocks_per_cu = bpc >= 0 ? bpc : tuned && preset.stage ? preset.blocks_per_cu : table_bpc;
       a.perm = A->d_perm;
       a.st_ivptr = S->d_ivptr;
       a.st_iv = S->d_iv;

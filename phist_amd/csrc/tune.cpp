@@ -10,15 +10,21 @@
 //   * per block width, the workgroups per CU of the persistent grid (the
 //     number of waves in flight, which trades latency hiding against the L2
 //     footprint of the gathered x rows);
-//   * per block width, for rows of 9 to 23 entries, the depth: 8 or 16
-//     entries of a row whose index loads and gathers go out together;
+//   * per block width, where the plain product runs the kernel's instance
+//     without epilogues, the depth: 8 or 16 entries of a row whose index loads
+//     and gathers go out together;
 //   * per block width above 16 columns, launches of 16 (and above 32, of 32)
 //     columns instead of one: each reads the matrix again, but gathers rows
 //     of x half (a quarter) as wide, so fewer of them leave L2;
 //   * per block width, where every workgroup tile's x window fits LDS, the
 //     product that stages each tile's window in LDS and gathers from there.
+// The launch is chosen twice per block width, for y = A x and for products
+// with an epilogue (timed on the shifted product): they run two instances of
+// the kernel whose best launches differ (600 k rows x 20 in a band of +-50k,
+// 16 FP32 columns: the plain product's choice made the shifted one 108 -> 180
+// us).  The library's own rule is kept unless another launch beats it.
 // The choice is stored on the matrix (SparseMat::tuned, used by every later
-// SpMV of that width unless a global setting overrides it) and cached for
+// SpMV of that width and kind unless a global setting overrides it) and cached for
 // the process by a matrix signature (scalar size, rows, entries, longest row,
 // a bucket of the mean distance of entries from the diagonal, block width),
 // so a matrix of the same signature is set up without timing again.
@@ -53,7 +59,7 @@ struct Signature {
 };
 struct Choice {
   int C, sigma;
-  SpmvTuned launch;
+  SpmvTuned launch, epilogue;  // of the product y = A x, and of products with an epilogue
 };
 std::map<Signature, Choice>& cache() {
   static std::map<Signature, Choice> c;
@@ -99,23 +105,28 @@ struct TrialBlock {
   TrialBlock& operator=(const TrialBlock&) = delete;
 };
 
-// fastest of reps products y = A x after one untimed launch; lb/bpc/depth < 0
-// take the library's usual choice (global settings, tuned entry, table)
+// fastest of reps products after one untimed launch: y = A x, or with
+// epilogue the shifted product (y = A x + y where A is not square); lb/bpc/
+// depth < 0 take the library's usual choice (global settings, tuned entry, rule)
 template <typename T>
-double time_product(const SparseMat<T>* A, Mvec<T>* x, Mvec<T>* y, int lb, int bpc, int depth, int reps,
-                    int col_block = -1, int stage = -1) {
+double time_product(const SparseMat<T>* A, bool epilogue, Mvec<T>* x, Mvec<T>* y, int lb, int bpc, int depth,
+                    int reps, int col_block = -1, int stage = -1) {
   Runtime& r = rt();
   SpmvRequest rq;
+  rq.has_shift = epilogue && A->nrows == A->ncols;
+  rq.has_beta = epilogue && !rq.has_shift;
+  const std::vector<T> shifts(rq.has_shift ? x->nvec : 0, T(0));
+  const T beta = rq.has_beta ? T(1) : T(0);
   rq.lane_bytes = lb;
   rq.blocks_per_cu = bpc;
   rq.depth = depth;
   rq.col_block = col_block;
   rq.stage = stage;
-  spmv_launch<T>(A, T(1), nullptr, x, T(0), y, rq, nullptr, nullptr);
+  spmv_launch<T>(A, T(1), shifts.data(), x, beta, y, rq, nullptr, nullptr);
   double best = 1e300;
   for (int k = 0; k < reps; k++) {
     PHX_HIP(hipEventRecord(r.ev_start, r.stream));
-    spmv_launch<T>(A, T(1), nullptr, x, T(0), y, rq, nullptr, nullptr);
+    spmv_launch<T>(A, T(1), shifts.data(), x, beta, y, rq, nullptr, nullptr);
     PHX_HIP(hipEventRecord(r.ev_stop, r.stream));
     PHX_HIP(hipEventSynchronize(r.ev_stop));
     float ms = 0.f;
@@ -125,14 +136,21 @@ double time_product(const SparseMat<T>* A, Mvec<T>* x, Mvec<T>* y, int lb, int b
   return best;
 }
 
+// The rule's own launch stays unless another one beats it by more than the
+// timing tells apart (3 % and a microsecond).
 template <typename T>
-SpmvTuned search_launch(const SparseMat<T>* A, int nvec, int reps) {
+SpmvTuned search_launch(const SparseMat<T>* A, int nvec, bool epilogue, int reps) {
   TrialBlock<T> x(A->col_map, A->ncols, nvec), y(A->row_map, A->nrows, nvec);
+  bool full = false;
+  SpmvTuned rule = spmv_rule_launch(A, nvec, epilogue, &full);
+  rule.ms = time_product<T>(A, epilogue, &x.v, &y.v, rule.lane_bytes, rule.blocks_per_cu, rule.depth, reps,
+                            rule.col_block, 0);
+  if (rule.blocks_per_cu == 0) rule.blocks_per_cu = 8;  // all that fit: a CU holds eight of these workgroups
   SpmvTuned best;
   best.ms = 1e300;
   std::vector<int> seen;
   std::vector<int> depths{8};
-  if (A->max_row_len > 8 && A->nnz < 24 * A->nrows) depths.push_back(16);  // (long rows run depth 8)
+  if (A->max_row_len > 8 && !full) depths.push_back(16);
   std::vector<int> blocks{0};
   for (int w : {16, 32})
     if (nvec > w) blocks.push_back(w);
@@ -150,11 +168,11 @@ SpmvTuned search_launch(const SparseMat<T>* A, int nvec, int reps) {
         std::vector<int> tried;
         for (int d : depths) {
           const int depth = stg ? (d >= 16 && vpl * (int)sizeof(T) <= 32 ? 16 : 8)
-                                : spmv_effective_depth(d, vpl, (int)sizeof(T), ncol);
+                                : spmv_effective_depth(d, vpl, (int)sizeof(T), ncol, full);
           if (std::find(tried.begin(), tried.end(), depth) != tried.end()) continue;
           tried.push_back(depth);
           for (int bpc : {1, 2, 3, 4, 6, 8}) {
-            const double ms = time_product<T>(A, &x.v, &y.v, lb, bpc, depth, reps, cbw, stg);
+            const double ms = time_product<T>(A, epilogue, &x.v, &y.v, lb, bpc, depth, reps, cbw, stg);
             if (ms < best.ms) {
               best.ms = ms;
               best.lane_bytes = lb;
@@ -168,7 +186,7 @@ SpmvTuned search_launch(const SparseMat<T>* A, int nvec, int reps) {
       }
     }
   }
-  return best;
+  return best.ms < rule.ms - std::max(0.03 * rule.ms, 1e-3) ? best : rule;
 }
 
 }  // namespace
@@ -190,7 +208,7 @@ void sparse_tune(SparseMat<T>* A, int n_nvec, const int* nvecs, int flags, doubl
   A->tuned.clear();
   for (int i = 0; i < n_nvec; i++) {
     TrialBlock<T> x(A->col_map, A->ncols, nvecs[i]), y(A->row_map, A->nrows, nvecs[i]);
-    const double ms = time_product<T>(A, &x.v, &y.v, -1, -1, -1, reps);
+    const double ms = time_product<T>(A, false, &x.v, &y.v, -1, -1, -1, reps);
     if (default_ms) default_ms[i] = ms;
   }
 
@@ -229,7 +247,7 @@ void sparse_tune(SparseMat<T>* A, int n_nvec, const int* nvecs, int flags, doubl
       std::vector<Choice> here(n_nvec);
       double total = 0.0;
       for (int i = 0; i < n_nvec; i++) {
-        here[i] = Choice{A->C, A->sigma, search_launch<T>(A, nvecs[i], reps)};
+        here[i] = Choice{A->C, A->sigma, search_launch<T>(A, nvecs[i], false, reps), SpmvTuned()};
         total += here[i].launch.ms;
       }
       if (total < best_total) {
@@ -237,16 +255,22 @@ void sparse_tune(SparseMat<T>* A, int n_nvec, const int* nvecs, int flags, doubl
         chosen = here;
       }
     }
-    std::lock_guard<std::mutex> lk(cache_mutex());
-    for (int i = 0; i < n_nvec; i++) cache()[sig[i]] = chosen[i];
   }
 
   if (chosen[0].C != A->C || chosen[0].sigma != A->sigma) sell_rebuild(A, chosen[0].C, chosen[0].sigma);
-  for (int i = 0; i < n_nvec; i++) A->tuned[nvecs[i]] = chosen[i].launch;
+  if (!hit) {
+    for (int i = 0; i < n_nvec; i++) chosen[i].epilogue = search_launch<T>(A, nvecs[i], true, reps);
+    std::lock_guard<std::mutex> lk(cache_mutex());
+    for (int i = 0; i < n_nvec; i++) cache()[sig[i]] = chosen[i];
+  }
+  for (int i = 0; i < n_nvec; i++) {
+    A->tuned[{nvecs[i], false}] = chosen[i].launch;
+    A->tuned[{nvecs[i], true}] = chosen[i].epilogue;
+  }
   for (int i = 0; i < n_nvec; i++) {
     TrialBlock<T> x(A->col_map, A->ncols, nvecs[i]), y(A->row_map, A->nrows, nvecs[i]);
-    const double ms = time_product<T>(A, &x.v, &y.v, -1, -1, -1, reps);
-    A->tuned[nvecs[i]].ms = ms;
+    const double ms = time_product<T>(A, false, &x.v, &y.v, -1, -1, -1, reps);
+    A->tuned[{nvecs[i], false}].ms = ms;
     if (tuned_ms) tuned_ms[i] = ms;
     if (settings) {
       settings[7 * i + 0] = A->C;

@@ -323,3 +323,34 @@ def test_spmv_stage_tuned_laplacian(be64):
         y.delete()
     A.delete()
     m.delete()
+
+
+def test_tune_keeps_the_shifted_product(be32):
+    """products with an epilogue have settings of their own: tuning a width
+    leaves the shifted product, whose best launch is not the plain one's, as
+    fast as it was (a quarter for the timing) and bit for bit the same"""
+    import time
+    n, k = 600000, 16
+    A = be32.banded_random(n, 20, 50000, 40.0, 3)
+    m = be32.map(n)
+    x, y = be32.mvec(m, k, np.random.default_rng(2).uniform(-1, 1, (n, k)).astype(np.float32)), be32.mvec(m, k)
+    sh = np.linspace(-1, 1, k).astype(np.float32)
+
+    def timed():
+        best = np.inf
+        for _ in range(6):
+            be32.synchronize()
+            t = time.perf_counter()
+            for _ in range(20):
+                be32.spmv_shifted(1.0, A, sh, x, 0.0, y)
+            be32.synchronize()
+            best = min(best, time.perf_counter() - t)
+        return best, y.get()
+
+    before, Y0 = timed()
+    _tune(be32, A, [k], 2)
+    after, Y1 = timed()
+    assert np.array_equal(Y0, Y1)
+    assert after <= 1.25 * before, (before, after)
+    for o in (x, y, A, m):
+        o.delete()
