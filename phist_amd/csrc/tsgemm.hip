@@ -724,7 +724,11 @@ __global__ void __launch_bounds__(kBlock) k_rowmix(const MixArgs<T> p) {
 // values sit in the MFMA result layout, which is the operand layout of a
 // Gram step over the same four rows, so the product needs no extra traffic
 // for W.
-template <typename T, int KS, int TM, int RT, int GRAM = 0, int TV = 1>
+//
+// EARLY: W's old values (mode 0, beta != 0) are requested with V's, for the
+// registers they take until the stores; without it each is read where it is
+// added (early_mix).
+template <typename T, int KS, int TM, int RT, int GRAM = 0, int TV = 1, bool EARLY = true>
 __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
   using M = Mfma<T>;
   constexpr int TG = GRAM == 1 ? TM : TV;  // tiles of the Gram's left operand
@@ -754,9 +758,9 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
   // are disjoint and each row's stores follow its own loads)
   constexpr int UNR = (GRAM == 0 && KS * TM <= 16) ? 2 : 1;
   const TileWalk tw = xcd_tiles(p.ntiles);
-  const bool upd = p.mode == 0 && p.beta != T(0);  // W's old values, requested with V's
+  const bool upd = p.mode == 0 && p.beta != T(0);
   for (int64_t t0 = tw.t; t0 < tw.end; t0 += UNR * tw.stride) {
-  T au[UNR][RT][KS], wold[UNR][RT][TM][4];
+  T au[UNR][RT][KS], wold[EARLY ? UNR : 1][RT][TM][4];
 #pragma unroll
   for (int u = 0; u < UNR; u++) {
     const int64_t tu = t0 + u * tw.stride;
@@ -781,7 +785,7 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
         for (int st = 0; st < KS; st++) au[u][rt_][st] = (tok && ra < p.nrows && j0 + st < p.k) ? vp[st] : T(0);
       }
     }
-    if (upd) {
+    if (EARLY && upd) {
 #pragma unroll
       for (int rt_ = 0; rt_ < RT; rt_++)
 #pragma unroll
@@ -790,7 +794,7 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
           for (int r = 0; r < 4; r++) {
             const int64_t row = r0 + rt_ * 16 + M::row(lane, r);
             const int c = tm * 16 + cc;
-            wold[u][rt_][tm][r] = (tok && row < p.nrows && c < p.m) ? p.w[row * p.ldw + c] : T(0);
+            wold[EARLY ? u : 0][rt_][tm][r] = (tok && row < p.nrows && c < p.m) ? p.w[row * p.ldw + c] : T(0);
           }
     }
   }
@@ -820,7 +824,7 @@ __global__ void __launch_bounds__(kBlock) k_rowmix_mfma(const MixArgs<T> p) {
           if (row < p.nrows && c < p.m) {
             T* wp = p.w + row * p.ldw + c;
             T val = acc[rt_][tm][r];
-            if (upd) val = fma(p.beta, wold[u][rt_][tm][r], val);
+            if (upd) val = fma(p.beta, EARLY ? wold[EARLY ? u : 0][rt_][tm][r] : *wp, val);
             *wp = val;
             acc[rt_][tm][r] = val;  // the Gram epilogue uses the stored values
           }
@@ -905,10 +909,25 @@ void mix_lpr(MixArgs<T>& p, int lpr, size_t lds) {
 constexpr size_t kMixLds = 32 * 1024;
 
 // one launch; the caller guarantees the LDS footprint fits and m <= 64*VPL
+// Whether W's old values are requested early.  They pay wherever W is read
+// (400 k rows, FP64, 64 -> 64 columns, beta 0.5: 208 us late, 145 early), but
+// not beside 16 scalar loads a lane (65 -> 1 columns: 69 late, 77 early).  Where
+// W is not read the two instances differ by their registers alone: few columns
+// of V to wide outputs want the late one (12 -> 48 columns 36 against 44, with
+// the Gram of 17 columns, 2.7 M rows, 179 against 206), the others run up to
+// 20 % faster with fewer waves (48 -> 64 FP32 columns, 50 k rows: 32 late, 26).
+template <typename T, int KS, int TM>
+bool early_mix(const MixArgs<T>& p) {
+  if (p.mode == 0 && p.beta != T(0)) return !(sizeof(T) == 8 && p.k > 48 && !p.vvec && TM <= 2);
+  return !(KS <= 4 && TM >= 2);
+}
+
 template <typename T, int KS, int TM>
 void mix_mfma_launch(MixArgs<T>& p) {
   constexpr int RT = KS >= 8 ? 1 : 2;
   auto kern = k_rowmix_mfma<T, KS, TM, RT>;
+  if constexpr ((KS <= 4 && TM >= 2) || (sizeof(T) == 8 && KS == 16 && TM <= 2))
+    if (!early_mix<T, KS, TM>(p)) kern = k_rowmix_mfma<T, KS, TM, RT, 0, 1, false>;
   p.ntiles = (p.nrows + 64 * RT - 1) / (64 * RT);
   const int grid = persistent_blocks(kern, 0, p.ntiles);
   ktimer_begin();
@@ -931,6 +950,8 @@ template <typename T, int KS, int TM, int GRAM, int TV>
 int mix_gram_launch(MixArgs<T>& p) {
   constexpr int RT = KS >= 8 ? 1 : 2;
   auto kern = k_rowmix_mfma<T, KS, TM, RT, GRAM, TV>;
+  if constexpr (KS <= 4 && TM >= 2)
+    if (!early_mix<T, KS, TM>(p)) kern = k_rowmix_mfma<T, KS, TM, RT, GRAM, TV, false>;
   p.ntiles = (p.nrows + 64 * RT - 1) / (64 * RT);
   const int na = GRAM == 1 ? p.m : p.ngv;
   const size_t lds = sizeof(T) * na * p.m;

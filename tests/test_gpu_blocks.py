@@ -630,3 +630,43 @@ def test_reductions_by_width(be64, be32, n, dtype):
         for o in (x, y, C):
             o.delete()
     m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("k", [8, 9, 12, 15, 16, 17, 49, 64, 65])
+def test_wide_outputs(be64, be32, k, dtype):
+    """W = alpha V C + beta W from few columns to wide outputs and from a
+    wide unaligned block to few, and the same with W'W in one call, around the
+    column tiles, on blocks and on views that start unaligned"""
+    be = be64 if dtype == np.float64 else be32
+    eps = np.finfo(dtype).eps
+    n = 1021
+    rng = np.random.default_rng(k)
+    V = rng.uniform(-1, 1, (n, k + 1)).astype(dtype)
+    m = be.map(n)
+    vb = be.mvec(m, k + 1, V)
+    for j in (1, 16, 17, 32, 33, 48, 64):
+        S0 = rng.uniform(-1, 1, (k, j)).astype(dtype)
+        W0 = rng.uniform(-1, 1, (n, j)).astype(dtype)
+        S, Sd = be.sdmat(k, j, data=S0), S0.astype(float)
+        for ofs in (0, 1):
+            v, Vd = vb.view(ofs, ofs + k - 1), V[:, ofs:ofs + k].astype(float)
+            for beta in (0.0, 0.75):
+                want = -1.25 * Vd @ Sd + beta * W0
+                bound = (k + 8) * eps * (1.25 * np.abs(Vd) @ np.abs(Sd) + beta * np.abs(W0))
+                w = be.mvec(m, j, W0)
+                be.times_sdmat(-1.25, v, S, beta, w)
+                got = w.get()
+                assert np.all(np.abs(got - want) <= bound), (j, ofs, beta)
+                w.set(W0)
+                G = be.sdmat(j, j)
+                be.call("fused_mvsd_mvTmv", be.s(-1.25), v.h, S.h, be.s(beta), w.h, G.h)
+                got = w.get().astype(float)
+                assert np.all(np.abs(got - want) <= bound), (j, ofs, beta)
+                assert np.all(np.abs(G.get() - got.T @ got) <= (n + 2) * eps * (np.abs(got).T @ np.abs(got)))
+                w.delete()
+                G.delete()
+            v.delete()
+        S.delete()
+    vb.delete()
+    m.delete()
