@@ -505,17 +505,18 @@ def test_spmv_lane_widths_bitexact(be64, be32, dtype, nvec):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("kind", ["sheet", "stencil", "band12", "band30"])
+@pytest.mark.parametrize("kind", ["sheet", "stencil", "band12", "band20", "band30"])
 def test_spmv_widths_by_column(be64, be32, kind, dtype):
     """every block width runs each column's own sum: the columns of a block
     product equal the one-column products bit for bit, whole vectors and
-    ragged widths, rows of at most 4, of 7, 12 and 30 entries, plain and
+    ragged widths, rows of at most 4, of 7, 12, 20 and 30 entries, plain and
     shifted with beta, on whole blocks and on a column view that starts and
     ends unaligned; the columns next to the view stay as they were; the dots
     agree with the columns"""
     be = be64 if dtype == np.float64 else be32
     A = {"sheet": lambda: be.honeycomb(37, 23, 0, 0, 0, 1.0, 7), "stencil": lambda: be.laplace3d(13, 7, 9),
          "band12": lambda: be.banded_random(1001, 12, 60, 40.0, 5),
+         "band20": lambda: be.banded_random(999, 20, 90, 40.0, 9),
          "band30": lambda: be.banded_random(997, 30, 400, 40.0, 6)}[kind]()
     n, widest = A.nrows, 133
     rng = np.random.default_rng(17)

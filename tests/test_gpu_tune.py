@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as ol
+import phist_amd
 
 pytestmark = pytest.mark.gpu
 
@@ -99,14 +100,30 @@ def test_tune_fp32_twin(be64):
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("nvec", [1, 4, 8, 16])
 def test_spmv_depth_bitexact(be64, be32, dtype, nvec, lane_bytes):
-    """depths 16 and 32 (the next batch's indices prefetched; a whole 32-entry
-    row's gathers in flight) and depth 8 give the same product bit for bit, on rows of 32 entries, of 40 entries (the
-    second batch of a row mostly empty) and of at most 7 (a 3D Laplacian:
-    every batch mostly empty), and agree with the oracle"""
+    """depths 8 and 16 (32 runs as 16) give the same plain product bit for bit:
+    on rows of 17, 20 and 23 entries (two batches at depth 16, three at 8), of
+    1 to 40 entries below 24 on average, of 32 and 40 entries (whose products
+    over scattered x rows run depth 8 alone where the matrix fills the chip)
+    and of at most 7 (a 3D Laplacian: one batch mostly empty), and agree with
+    the oracle"""
     be = be64 if dtype == np.float64 else be32
     fl = ctypes.c_int(0)
-    for n, nnz, hb in ((50000, 32, 3000), (30000, 40, 500), (8000, 0, 0)):
-        A = be.banded_random(n, nnz, hb, 40.0, 17 + nnz) if nnz else be.laplace3d(20, 20, 20)
+    rng = np.random.default_rng(7)
+    rows = [(np.sort(rng.choice(4000, 40 if i % 3 == 0 else 1 + i % 23, replace=False)), i) for i in range(4000)]
+    ctype = ctypes.c_double if dtype == np.float64 else ctypes.c_float
+
+    @phist_amd.ROWFUNC
+    def mixed(i, nnz, cols, vals, arg):
+        nnz[0] = len(rows[i][0])
+        v = ctypes.cast(vals, ctypes.POINTER(ctype))
+        for j, c in enumerate(rows[i][0]):
+            cols[j], v[j] = int(c), 0.25 + ((i + 3 * j) % 11) / 16
+        return 0
+
+    for n, nnz, hb in ((4000, -1, 0), (40000, 17, 2000), (40000, 20, 300), (30000, 23, 2000), (50000, 32, 3000),
+                       (30000, 40, 500), (8000, 0, 0)):
+        A = (be.banded_random(n, nnz, hb, 40.0, 17 + nnz) if nnz > 0 else be.laplace3d(20, 20, 20) if nnz == 0
+             else be.from_rowfunc(n, 40, mixed, None))
         ro, ci, va = A.crs()
         ref = ol.Crs(n, n, ro, ci, va.astype(float))
         m = be.map(n)
