@@ -137,7 +137,7 @@ def test_serve_graphs_bitexact(be64, graphs):
 def test_paired_updates_equal_single_ones(be64, k, iters):
     """the direction and solution updates of two iterations in one pass give
     bit for bit those of one pass per iteration (captured iterations do their
-    own), for even and odd numbers of iterations, whole vectors and ragged
+    own; the counters show that they ran), for even and odd numbers of iterations, whole vectors and ragged
     widths, FP64 and FP32, and with fewer slots than systems"""
     A = be64.honeycomb(31, 29, 0, 0, 0, 1.0, 7)
     n = A.nrows
@@ -147,11 +147,17 @@ def test_paired_updates_equal_single_ones(be64, k, iters):
     try:
         for graphs in (False, True):
             be64.set_minres_graphs(graphs, 1, 1)
+            c0, n0 = be64.minres_graph_stats()
             X, Y, Z = (be64.mvec(A.domain_map, k) for _ in range(3))
             be64.minres_shifted(A, shifts, B, X, 1e-13, iters)
             be64.minres_shifted(A, shifts, B, Y, 1e-13, iters, fp32=True)
             be64.minres_refill(A, shifts, B, Z, 1e-13, iters, max(1, k // 2))
             out[graphs] = [v.get() for v in (X, Y, Z)]
+            c1, n1 = be64.minres_graph_stats()
+            if graphs:  # three solves, every iteration of each replayed
+                assert c1 - c0 >= 3 and n1 - n0 >= 3 * iters, (c1 - c0, n1 - n0)
+            else:
+                assert (c1, n1) == (c0, n0)
             for v in (X, Y, Z):
                 v.delete()
     finally:
