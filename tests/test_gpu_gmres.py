@@ -159,13 +159,15 @@ def test_gmres_device_givens_matches_host(be64, restart, nsys, tol):
     A.delete()
 
 
+@pytest.mark.parametrize("fp32", [False, True])
 @pytest.mark.parametrize("restart,nsys", [(1, 3), (2, 1), (4, 64), (5, 33), (32, 2), (31, 5)])
-def test_gmres_two_sweep_cycle(be64, restart, nsys):
+def test_gmres_two_sweep_cycle(be64, restart, nsys, fp32):
     """the two-sweep cycle (second orthogonalisation one step late) against
     the host rotations' three sweeps around the sizes of its register slots
-    and system groups: iteration counts within one, the tolerance by the true
-    residual, for a band and for a diagonal of three values, whose Krylov
-    space ends after three steps"""
+    and system groups, in FP64 and in FP32, whose norms come from a difference
+    cut at a larger eps: iteration counts within one (FP32: a step a cycle),
+    the tolerance by the true residual, for a band and for a diagonal of three
+    values, whose Krylov space ends after three steps"""
     import ctypes
 
     import phist_amd
@@ -187,15 +189,17 @@ def test_gmres_two_sweep_cycle(be64, restart, nsys):
             for dev in (0, 1):
                 be64.L.phist_amd_set_gmres_device(dev, ctypes.byref(fl))
                 B, X = be64.mvec(A.domain_map, nsys, Bh), be64.mvec(A.domain_map, nsys)
-                it, rr, unconv = be64.gmres_shifted(A, shifts, B, X, 1e-9, 500, restart=restart)
+                tol = 1e-5 if fp32 else 1e-9
+                it, rr, unconv = be64.gmres_shifted(A, shifts, B, X, tol, 500, restart=restart, fp32=fp32)
                 assert unconv == 0
                 live = [j for j in range(nsys) if np.any(Bh[:, j])]
                 got = true_relres(A, shifts[live], Bh[:, live], X.get()[:, live])
-                assert np.all(got <= 2e-9), (dev, got)
-                its[dev] = it
+                assert np.all(got <= 2 * tol), (dev, got)
+                its[dev] = np.array(it)
                 B.delete()
                 X.delete()
         finally:
             be64.L.phist_amd_set_gmres_device(1, ctypes.byref(fl))
-        assert np.all(np.abs(its[0] - its[1]) <= 1), its
+        slack = 1 + its[0] // restart if fp32 else 1
+        assert np.all(np.abs(its[0] - its[1]) <= slack), its
         A.delete()
