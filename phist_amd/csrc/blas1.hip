@@ -41,7 +41,10 @@ enum : int { B_READX = 1, B_READY = 2 };
 constexpr int kRowUnroll = 4;
 static_assert(kRowUnroll == 4, "k_coldot adds four row sums");
 // workgroups per CU of the dots: with four rows under way per lane group four
-// keep HBM busy, and the partial sums are half as many as with eight
+// keep HBM busy, and the partial sums are half as many as with eight; two
+// blocks read in single FP64 columns by wide groups run best with three (2.7 M
+// rows, us at 3 / 4 / one row and eight: 17 columns 159 / 165 / 155, 33: 308 /
+// 319 / 289, 63: 464 / 480 / 439; 400 k, 33: 44 / 48 / 48)
 constexpr int kDotBlocksPerCu = 4;
 
 template <typename T, int VPL, int LPR>
@@ -187,7 +190,8 @@ int launch_kind(Kind kind, RowArgs<T>& p) {
       hipLaunchKernelGGL((k_elemwise<T, VPL, LPR>), dim3(grid), dim3(kBlock), 0, rt().stream, p);
       break;
     default:
-      grid = reducing_blocks(k_coldot<T, VPL, LPR>, 0, p.ntiles, kDotBlocksPerCu);
+      grid = reducing_blocks(k_coldot<T, VPL, LPR>, 0, p.ntiles,
+                             sizeof(T) == 8 && VPL == 1 && LPR >= 32 && p.x != p.y ? 3 : kDotBlocksPerCu);
       p.partials = (T*)device_work(sizeof(T) * ((size_t)grid * p.ncols + p.ncols));
       hipLaunchKernelGGL((k_coldot<T, VPL, LPR>), dim3(grid), dim3(kBlock), 0, rt().stream, p);
       break;
