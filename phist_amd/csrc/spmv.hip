@@ -287,8 +287,9 @@ __global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
 #pragma unroll
         for (int kk = 0; kk < SUB; kk++) {
           const int k = k0 + kk;
-          if constexpr (!AHEAD) xoff[kk] = offset(group_bcast<LPR>(cj[k / LPR], k % LPR, lane));
-          if (colok && (j0 + k) < cur.w) gather(xoff[kk], xg[kk]);
+          int32_t cc = 0;
+          if constexpr (!AHEAD) cc = group_bcast<LPR>(cj[k / LPR], k % LPR, lane);
+          if (colok && (j0 + k) < cur.w) gather(AHEAD ? xoff[kk] : offset(cc), xg[kk]);
         }
 #pragma unroll
         for (int kk = 0; kk < SUB; kk++) {
@@ -897,24 +898,27 @@ inline bool spmv_long_rows(const SparseMat<T>* A) {
 // What the x rows of a product with nvec columns cost to gather, from the
 // rows' bytes and a sample of the entries.  few: the row groups leave the
 // chip at no more than two waves per SIMD, whose latency nothing covers.
-// near: neighbouring rows gather neighbouring x rows (a stencil, a chain).
+// spread: the x rows are columns of a wider block, each on cache lines of its
+// own, which count instead of its bytes.  near: neighbouring rows gather
+// neighbouring x rows (a stencil, a chain) that share lines.
 // window: bytes of x within reach of neighbouring rows; up to 16 KB (local)
 // they stay in the L1, and from 512 KB (wide) on they are a share of the L2.
 struct SpmvReach {
   int rb;  // bytes of an x row
   double window;
-  bool few, near, local, wide;
+  bool few, spread, near, local, wide;
   bool scattered() const { return !few && !near && !local; }
 };
 template <typename T>
-SpmvReach spmv_reach(const SparseMat<T>* A, int nvec) {
+SpmvReach spmv_reach(const SparseMat<T>* A, int nvec, int64_t ldx) {
   SpmvReach r;
   r.rb = nvec * (int)sizeof(T);
+  r.spread = ldx > nvec && ldx * (int64_t)sizeof(T) > 128;
   int lanes = 1;
   while (lanes * 16 < r.rb && lanes < 64) lanes <<= 1;
   r.few = A->nrows * lanes <= (int64_t)rt().num_cu * 512;
-  r.near = A->gather_next >= 0.5;
-  r.window = 4.0 * A->gather_span * r.rb;
+  r.near = A->gather_next >= 0.5 && !r.spread;
+  r.window = 4.0 * A->gather_span * (r.spread ? (r.rb + 127) / 128 * 128 : r.rb);
   r.local = r.window <= 16.0 * 1024.0;
   r.wide = r.window >= 512.0 * 1024.0;
   return r;
@@ -928,6 +932,7 @@ SpmvReach spmv_reach(const SparseMat<T>* A, int nvec) {
 // in +-2000 106 / 87, 30 k 22 / 18, 4000 rows 17 / 6, 64 columns 33 / 7)
 inline bool spmv_col_blocks(const SpmvReach& r, int64_t nrows) {
   const double mib = 1024.0 * 1024.0, block = (double)nrows * r.rb;
+  if (r.spread) return r.rb > 128 && !r.few;
   return r.rb > 128 && ((r.window >= 4.0 * mib && block >= 32.0 * mib) || (!r.wide && block >= 128.0 * mib));
 }
 
@@ -976,9 +981,8 @@ bool spmv_full_instance(const SparseMat<T>* A, const SpmvReach& r, bool needs) {
 //    lanes; 12 columns, 96 bytes: 466 / 475), else b6 (5 columns: 45 at b6,
 //    55 at b4)
 template <typename T>
-SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
+SpmvTuned spmv_default_launch(const SparseMat<T>* A, const SpmvReach& r, bool full) {
   SpmvTuned d;
-  const SpmvReach r = spmv_reach(A, nvec);
   const int rb = r.rb;
   d.blocks_per_cu = 0;
   if (spmv_long_rows(A)) {
@@ -986,7 +990,7 @@ SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
     if (cols) d.col_block = 128 / (int)sizeof(T);
     d.lane_bytes = rb >= 128 && !r.few ? 32 : 0;
     d.depth = !r.few ? 8 : 16;
-    if (r.wide && !r.few) d.blocks_per_cu = rb <= 8 ? 1 : rb <= 32 ? 3 : rb > 128 && !cols && full ? 2 : 0;
+    if (r.wide && !r.few) d.blocks_per_cu = rb <= 8 ? 1 : rb <= 32 ? 3 : rb > 128 && rb % 32 == 0 && !cols && full ? 2 : 0;
   } else if (A->max_row_len > 8) {
     if (full) {
       const bool chain = r.near && r.wide, near_full = r.local && A->nnz >= 16 * A->nrows;
@@ -998,7 +1002,7 @@ SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
     }
   } else if (A->max_row_len > 4) {
     const bool last_level = (double)A->nrows * rb < 128.0 * 1024.0 * 1024.0;  // x fits its share of that cache
-    const bool one_lane = rb == 32 && r.near && A->nrows >= (int64_t)rt().num_cu * 512;
+    const bool one_lane = rb == 32 && (r.near || r.spread) && A->nrows >= (int64_t)rt().num_cu * 512;
     d.lane_bytes = one_lane || rb >= 256 || (full && rb >= 128 && !r.few && last_level) ? 32 : 0;
     d.blocks_per_cu = rb >= (full ? 128 : 64) ? 4 : 6;
   } else {
@@ -1010,9 +1014,10 @@ SpmvTuned spmv_default_launch(const SparseMat<T>* A, int nvec, bool full) {
 
 template <typename T>
 SpmvTuned spmv_rule_launch(const SparseMat<T>* A, int nvec, bool epilogue, bool* full) {
-  const bool f = spmv_full_instance(A, spmv_reach(A, nvec), epilogue);
+  const SpmvReach r = spmv_reach(A, nvec, nvec);
+  const bool f = spmv_full_instance(A, r, epilogue);
   if (full) *full = f;
-  return spmv_default_launch(A, nvec, f);
+  return spmv_default_launch(A, r, f);
 }
 template SpmvTuned spmv_rule_launch<double>(const SparseMat<double>*, int, bool, bool*);
 template SpmvTuned spmv_rule_launch<float>(const SparseMat<float>*, int, bool, bool*);
@@ -1048,10 +1053,10 @@ void spmv_launch(const SparseMat<T>* A, T alpha, const T* shifts_host, const Mve
   if (y) vec_ok = vec_ok && (y->lda % V16 == 0) && aligned16(y->dev());
   if (req.axpy_u) vec_ok = vec_ok && (U->lda % V16 == 0) && aligned16(U->dev());
   const bool needs = req.has_shift || req.has_beta || req.dot_ww || req.dot_vw || req.axpy_u || req.xscale;
-  const SpmvReach reach = spmv_reach(A, nvec);
+  const SpmvReach reach = spmv_reach(A, nvec, x->lda);
   const bool full = spmv_full_instance(A, reach, needs);
   const auto tuned_at = A->tuned.find({nvec, needs});
-  const SpmvTuned preset = tuned_at != A->tuned.end() ? tuned_at->second : spmv_default_launch(A, nvec, full);
+  const SpmvTuned preset = tuned_at != A->tuned.end() ? tuned_at->second : spmv_default_launch(A, reach, full);
   // x rows of each tile staged in LDS (where the matrix's tiles allow it)
   int stage = req.stage;
   if (stage < 0) stage = rt().spmv_stage;
