@@ -980,6 +980,10 @@ bool spmv_full_instance(const SparseMat<T>* A, const SpmvReach& r, bool needs) {
 //    32-byte lanes, b3 (8 M rows, 32 columns: 1092 against 1470 in 16-byte
 //    lanes; 12 columns, 96 bytes: 466 / 475), else b6 (5 columns: 45 at b6,
 //    55 at b4)
+//  - up to 16 bytes of each row of a wider block, shifted: b2 (1 of 40 columns,
+//    FP64, 100^3 Laplacian 83 against 93 as many as fit, sheet 31 / 34, 600 k x
+//    20 in +-50k 160 / 167); two columns in a lane each, b3 (FP64 83 / 89, 30 /
+//    35, 121 / 168)
 template <typename T>
 SpmvTuned spmv_default_launch(const SparseMat<T>* A, const SpmvReach& r, bool full) {
   SpmvTuned d;
@@ -1002,12 +1006,17 @@ SpmvTuned spmv_default_launch(const SparseMat<T>* A, const SpmvReach& r, bool fu
     }
   } else if (A->max_row_len > 4) {
     const bool last_level = (double)A->nrows * rb < 128.0 * 1024.0 * 1024.0;  // x fits its share of that cache
-    const bool one_lane = rb == 32 && (r.near || r.spread) && A->nrows >= (int64_t)rt().num_cu * 512;
+    const bool one_lane = rb == 32 && (r.near || (r.spread && !full)) && A->nrows >= (int64_t)rt().num_cu * 512;
     d.lane_bytes = one_lane || rb >= 256 || (full && rb >= 128 && !r.few && last_level) ? 32 : 0;
     d.blocks_per_cu = rb >= (full ? 128 : 64) ? 4 : 6;
   } else {
     d.lane_bytes = rb >= 128 ? 32 : 0;
     d.blocks_per_cu = rb >= 128 ? 3 : 6;
+  }
+  if (r.spread && full && rb <= 16) {
+    const bool two = rb == 2 * (int)sizeof(T);
+    if (two) d.lane_bytes = (int)sizeof(T);
+    d.blocks_per_cu = two ? 3 : 2;
   }
   return d;
 }
