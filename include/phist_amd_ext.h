@@ -38,15 +38,15 @@ void phist_amd_set_spmv_lane_bytes(int bytes, int* iflag);
 /* entries of a row whose val/col loads and x gathers the SpMV issues
  * together before their multiply-adds (0 = the default: the matrix's tuned
  * value, else 8 or 16 by a rule; 8, 16 or 32).  16 (and 32, the same) applies
- * to plain products of rows shorter than 24 entries, in row groups of at most
- * 8 lanes gathering at most 32 bytes each; elsewhere 8, and 4 for matrices
- * whose longest row has at most 4 entries.  Every choice gives the same
+ * to products without an epilogue (not to those of long rows over scattered x
+ * rows), in row groups of at most 8 lanes gathering at most 32 bytes each;
+ * elsewhere 8, and 4 for matrices whose longest row has at most 4 entries.  Every choice gives the same
  * result bit for bit. */
 void phist_amd_set_spmv_depth(int slots, int* iflag);
-/* block columns per SpMV launch: ncols > 0 = at most that many (a multiple of
+/* block columns per SpMV launch (at most 256): ncols > 0 = at most that many (a multiple of
  * the scalars each lane holds, else ignored), 0 = as many as 64 lane groups
  * hold, -1 = the default: the matrix's tuned value, else 128 bytes of columns
- * for rows of at least 24 entries and 0 for shorter ones.  Each further
+ * for rows of at least 24 entries whose x rows exceed the caches, 0 for others.  Each further
  * launch reads the matrix again; wide rows of x (256-byte rows at 32 FP64
  * columns) gather half as many bytes per launch in two blocks of 16.  Every
  * choice gives the same result bit for bit (column dots to rounding). */

@@ -102,13 +102,12 @@ struct Runtime {
   int sell_C = 0, sell_sigma = 0;
   // maximum persistent grid size for streaming kernels (0 = automatic)
   int grid_blocks = 0;
-  // workgroups per CU for the SpMV: the x gathers of a +-band thrash L2 when
-  // too many rows are in flight, two workgroups per CU measured best
-  int spmv_blocks_per_cu = -1;  // < 0: spmv_table_blocks_per_cu
-  // bytes of a block row each SpMV lane gathers per nonzero (0: one 16-byte vector)
+  // workgroups per CU for the SpMV (< 0: the matrix's tuned value, else the rule of spmv.hip)
+  int spmv_blocks_per_cu = -1;
+  // bytes of a block row each SpMV lane gathers per nonzero (0: the matrix's tuned value, else the rule)
   int spmv_lane_bytes = 0;
   // entries per row whose val/col loads and x gathers the SpMV issues
-  // together (8 or 32; < 0: the matrix's tuned value, else 8)
+  // together (8 or 16; < 0: the matrix's tuned value, else the rule)
   int spmv_depth = -1;
   // y of the SpMV written with non-temporal stores, which keeps L2 for the
   // gathered x rows: 1 always, 0 never, -1 (default) when y spans at least
@@ -116,8 +115,8 @@ struct Runtime {
   // there) and its rows are shorter than a 128-byte line (measured: rows of
   // 32 and 64 bytes gain 1 %, rows of 128 and 256 bytes lose 4-5 %)
   int spmv_nt_y = -1;
-  // block columns per SpMV launch: > 0 at most that many, 0 as many as 64
-  // lane groups hold, -1 (default) the matrix's tuned value
+  // block columns per SpMV launch: > 0 at most that many, 0 as many as one
+  // launch holds, -1 (default) the matrix's tuned value, else the rule
   int spmv_col_block = -1;
   // x rows of each workgroup tile staged in LDS before the tile's gathers
   // (matrices whose tiles gather from a few short column intervals): 1 on

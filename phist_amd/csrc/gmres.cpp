@@ -22,10 +22,10 @@
 // norm follows from ||w||^2 - ||V'w||^2, and since A V = V H the product's
 // missing correction only changes the coefficients, h(0:i) -= H e.  The
 // sweeps are bound by the basis they read (2.1 M rows, 16 systems, FP64, 30
-// steps: 98.4 ms in three sweeps and a normalisation per step, 72.1 ms in two;
-// 5.1 TB/s in the sweeps).
-// (for more than 64 systems or m > 32: a Gram and a row mix of the whole
-// basis per pass, of which only the blocks' diagonals are used).
+// steps: 98.4 ms in three sweeps and a normalisation per step, 72.1 ms in two
+// and 65.5 with the basis read non-temporally; 5.1-5.4 TB/s in the sweeps).
+// More than 64 systems or m > 32 take a Gram and a row mix of the whole basis
+// per pass, of which only the blocks' diagonals are used.
 //   Givens rotations of every system's Hessenberg column on the device (one
 //   thread per system; on the host for the whole-basis passes); the
 //   implicit residual |g_{i+1}| decides convergence.

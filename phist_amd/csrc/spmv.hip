@@ -163,8 +163,8 @@ __device__ inline T group_bcast_t(T v, int src, int lane) {
 // 1968 -> 1092; 24-spin chain, 4 FP32 columns 147 -> 106, 1 FP64 column 153 ->
 // 121; 128^3 Laplacian, 1 column 51.8 -> 40.4, 16 columns 225 -> 213; 4.2 M
 // rows x 32 in a band of +-50k, 8 columns 1242 -> 1001, 32 columns 4962 ->
-// 3280 (floors by the byte model at 5.5 TB/s: 35, 815, 68, 86, 38, 129, 390
-// and 683).
+// 3280 (bytes each call cannot do without at 5.88 TB/s, the card's read rate:
+// 33, 762, 64, 80, 36, 121, 365 and 639).
 //
 // AHEAD: the x offsets of a batch are settled before its first gather.
 // Without it the compiler of the epilogue instance forms each offset in a
@@ -374,9 +374,8 @@ __global__ void __launch_bounds__(kBlock) k_spmv(const SpmvArgs<T> a) {
 // cooperatively (lane q takes slot j = jb*LPR + q, coalesced over the rows
 // of the chunk) and share them by group broadcast, so every index is read
 // from memory once.  A batch covers SL entries of each row (the depth: 8, or
-// 32 for long rows): its KB = SL/LPR val/col loads per lane, then all its x
-// gathers, go out before the first FMA of the batch, so a row of 32 entries
-// costs one round trip for its indices and one for its gathers.
+// 16 for staged products): its KB = SL/LPR val/col loads per lane, then its x
+// gathers, go out before the first FMA of the batch.
 //
 // STG: before a tile's rows, the workgroup copies the x rows the tile
 // gathers from (its column intervals, each taken by one wave with 16-byte
@@ -398,10 +397,7 @@ __global__ void __launch_bounds__(kBlock) k_sell_spmv(const SpmvArgs<T> a) {
   constexpr int RPB = (kBlock / 64) * RPW;
   constexpr int KB = SL > LPR ? SL / LPR : 1;  // val/col loads per lane and batch
   constexpr int BATCH = KB * LPR;              // slots per batch and row
-  // gathers issued before their FMAs: up to 32 at depth 32 with at most 16
-  // gathered bytes per lane, otherwise 16 (register budget)
-  constexpr int SUBMAX = (SL >= 32 && VPL * (int)sizeof(T) <= 16) ? 32 : 16;
-  constexpr int SUB = BATCH < SUBMAX ? BATCH : SUBMAX;  // gathers issued before their FMAs
+  constexpr int SUB = BATCH < 16 ? BATCH : 16;  // gathers issued before their FMAs (register budget)
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
   const int q = lane % LPR;
