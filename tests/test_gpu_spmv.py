@@ -683,3 +683,48 @@ def test_spmv_launch_rules(be64, be32, kind, widths, dtype):
         y.delete()
     A.delete()
     m.delete()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["sheet", "stencil", "band20", "band30"])
+def test_spmv_views_of_a_wide_block(be64, be32, kind, dtype):
+    """columns of a block of 40 and 41, each row on cache lines of its own,
+    have launches of their own: the compact block's product bit for bit,
+    plain and shifted with beta, dots that agree with it, and the columns
+    beside the view as they were"""
+    be = be64 if dtype == np.float64 else be32
+    A = {"sheet": lambda: be.honeycomb(301, 299, 0, 0, 0, 1.0, 7), "stencil": lambda: be.laplace3d(53, 52, 51),
+         "band20": lambda: be.banded_random(30001, 20, 7000, 40.0, 5),
+         "band30": lambda: be.banded_random(40001, 30, 3000, 40.0, 6)}[kind]()
+    n = A.nrows
+    rng = np.random.default_rng(31)
+    m = be.map(n)
+    eps = np.finfo(dtype).eps
+    for k, ld, ofs in ((1, 41, 0), (1, 40, 1), (2, 40, 0), (2, 41, 39), (4, 40, 4), (4, 41, 1), (5, 40, 0), (8, 40, 3),
+                       (33, 41, 2)):
+        X, Y = (rng.uniform(-1, 1, (n, ld)).astype(dtype) for _ in range(2))
+        sh = rng.uniform(-2, 2, k).astype(dtype)
+        cols = slice(ofs, ofs + k)
+        x, y = be.mvec(m, k, X[:, cols]), be.mvec(m, k, Y[:, cols])
+        be.spmv_shifted(0.75, A, sh, x, -0.3, y)
+        shifted = y.get()
+        be.spmv(0.75, A, x, 0.0, y)
+        plain = y.get()
+        XB, YB = be.mvec(m, ld, X), be.mvec(m, ld, Y)
+        xv, yv = XB.view(ofs, ofs + k - 1), YB.view(ofs, ofs + k - 1)
+        be.spmv_shifted(0.75, A, sh, xv, -0.3, yv)
+        got, want = YB.get(), Y.copy()
+        want[:, cols] = shifted
+        assert np.array_equal(got, want), (k, ld, ofs)
+        be.spmv(0.75, A, xv, 0.0, yv)
+        want[:, cols] = plain
+        assert np.array_equal(YB.get(), want), (k, ld, ofs)
+        ww, vw = be.fused_spmv_mvdot(0.75, A, xv, 0.0, yv)
+        assert np.array_equal(YB.get(), want), (k, ld, ofs)
+        w, v = plain.astype(float), X[:, cols].astype(float)
+        assert np.all(np.abs(ww - (w * w).sum(0)) <= (n + 2) * eps * (w * w).sum(0)), (k, ld, ofs)
+        assert np.all(np.abs(vw - (v * w).sum(0)) <= (n + 2) * eps * np.abs(v * w).sum(0)), (k, ld, ofs)
+        for o in (xv, yv, XB, YB, x, y):
+            o.delete()
+    A.delete()
+    m.delete()
